@@ -27,8 +27,12 @@
  * (paged_attention.cu:199-200, 369-370): any head_dim up to 1024, any block
  * size up to 4096 and num_q_heads a multiple of num_kv_heads.  head_dim 64 /
  * 128 with block_size 16 and num_q_heads / num_kv_heads in {1, 2, 4, 8} run
- * the tuned kernels; every other shape runs a shape-general kernel (no
- * workspace; partition_size is ignored).  Cache writes accept any shape.
+ * the tuned kernels; every other shape runs the shape-general kernels
+ * (partition_size and the workspace argument are ignored; decode splits long
+ * contexts over library-owned scratch per (device, stream) and runs unsplit
+ * where there is none: during a capture on a stream that has no scratch yet,
+ * through rllm_paged_attention_decode_noalloc, or when no memory is left).
+ * Cache writes accept any shape.
  *
  * Differences from the reference kernels, all deliberate:
  *   - a sequence with seq_len <= 0 gets an all-zero output row (the reference

@@ -1575,7 +1575,7 @@ int32_t decode_impl(void* out, const void* q, const void* kc, const void* vc, co
     // (no workspace; partition_size does not apply)
     if (!specialised_shape(hq, hkv, d, bs))
         return generic_attention(out, q, kc, vc, bt, seq_lens, nullptr, num_seqs, num_seqs, hq, hkv, d, bs, maxb,
-                                 scale, q_dtype, kv_dtype, k_scale, v_scale, as_stream(stream));
+                                 scale, q_dtype, kv_dtype, k_scale, v_scale, !fixed_scratch, as_stream(stream));
     Kernels kern;
     RLLM_CHECK_ARG(pick_kernels(q_dtype, kv_dtype, d, G, &kern));
 

@@ -1,0 +1,101 @@
+"""The matrix-core kernels of the shape-general attention at the sizes where
+their tiles, windows and context parts end, over every form that selects a
+path, and rows whose values are not finite."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+import rllm_amd
+from gpu_util import f32, log_case, t16, ti
+from helpers import TOL_BF16, assert_close, random_case
+from rllm_amd import ops
+
+pytestmark = pytest.mark.gpu
+TORCH = {O.BF16: torch.bfloat16, O.F16: torch.float16}
+
+# (head_dim, q heads, kv heads, block size, kind, contexts): windows are 128
+# tokens, rounds 512, head_dim classes end at 64, 96, 128, 192, 256, a group
+# holds 16 heads
+DECODE = [
+    (128, 3, 1, 16, O.BF16, [1, 7, 8, 9, 15, 16, 17, 127, 128, 129]),
+    (128, 6, 2, 16, O.F16, [511, 512, 513, 1023, 1024, 1025, 2600]),
+    (96, 17, 1, 8, O.F16, [0, 130, 640]),
+    (72, 33, 1, 24, O.BF16, [0, 25, 700]),
+    (200, 5, 5, 40, O.F16, [1, 41, 513]),
+    (256, 20, 4, 64, O.BF16, [63, 65, 2049]),
+    (8, 2, 1, 32, O.BF16, [5, 33, 600]),
+]
+
+
+def _decode(dev, case, q, k, v, bt, sl, scale):
+    D, hq, hkv, bs, kind, _ = case
+    qb, kb, vb = O.encode(q, kind), O.encode(k, kind), O.encode(v, kind)
+    out = ops.paged_decode(t16(qb, TORCH[kind], dev), t16(kb, TORCH[kind], dev), t16(vb, TORCH[kind], dev),
+                           ti(bt, torch.int32, dev), ti(sl, torch.int32, dev), scale)
+    torch.cuda.synchronize()
+    return f32(out), O.paged_attention_decode(qb, kind, kb, vb, kind, bt, sl, scale, precision=1)
+
+
+@pytest.mark.parametrize("case", DECODE, ids=[f"D{c[0]}-{c[1]}x{c[2]}-bs{c[3]}" for c in DECODE])
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_decode_edges_vs_oracle(dev, case, sign):
+    D, hq, hkv, bs, kind, lens = case
+    rng = np.random.default_rng(D + hq)
+    q, k, v, bt, sl = random_case(rng, len(lens), hq, hkv, D, (max(lens), max(lens)), bs=bs, neg_blocks=1)
+    sl[:] = lens
+    log_case(f"generic mfma decode {case} sign {sign}")
+    got, ref = _decode(dev, case, q, k, v, bt, sl, sign / np.sqrt(D))
+    assert_close(got, ref, TOL_BF16, f"decode {case}")
+    # outputs keep the fp32 weights' precision: relative L2 within the output
+    # rounding (2^-9 / 2^-12 per element, uniform) and a factor 1.5
+    live = np.array(lens) > 0
+    rel = np.linalg.norm(got[live] - ref[live]) / np.linalg.norm(ref[live])
+    assert rel < 1.5 * (2.0 ** -9 if kind == O.BF16 else 2.0 ** -12), rel
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+@pytest.mark.parametrize("past", [True, False])
+def test_decode_values_that_are_not_finite(dev, bad, past):
+    # slots past the context are not read; an attended infinity or NaN reaches
+    # its own row and head_dim only, as a sum over the visible keys gives it
+    case = (128, 6, 2, 16, O.BF16, [40, 600])
+    rng = np.random.default_rng(5)
+    q, k, v, bt, sl = random_case(rng, 2, 6, 2, 128, (600, 600))
+    sl[:] = [40, 600]
+    pos = 40 if past else 17
+    v[bt[0, pos // 16], 1, 3, pos % 16] = bad
+    if past:
+        k[bt[0, pos // 16], 1, 3, pos % 16] = bad
+    log_case(f"generic mfma decode value {bad} past {past}")
+    got, ref = _decode(dev, case, q, k, v, bt, sl, 1 / np.sqrt(128))
+    assert np.array_equal(np.isfinite(got), np.isfinite(ref))
+    assert np.array_equal(np.isposinf(got), np.isposinf(ref))
+    ok = np.isfinite(ref)
+    assert ok.all() == past
+    assert (np.abs(got[ok] - ref[ok]) <= 2e-2 + 1e-2 * np.abs(ref[ok])).all()
+
+
+def test_decode_repeats_bitwise_and_unsplit_agrees(dev):
+    # context parts merge in order; a capture without scratch runs unsplit
+    case = (96, 24, 8, 16, O.BF16, None)
+    rng = np.random.default_rng(9)
+    q, k, v, bt, sl = random_case(rng, 4, 24, 8, 96, (100, 3000))
+    kind = O.BF16
+    args = (t16(O.encode(q, kind), TORCH[kind], dev), t16(O.encode(k, kind), TORCH[kind], dev),
+            t16(O.encode(v, kind), TORCH[kind], dev), ti(bt, torch.int32, dev), ti(sl, torch.int32, dev), 0.1)
+    log_case("generic mfma decode repeat")
+    a = ops.paged_decode(*args)
+    b = ops.paged_decode(*args)
+    out = torch.empty_like(a)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        ops.paged_decode(*args, out=out, validate=False)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_close(f32(out), f32(a), TOL_BF16, "unsplit")
+    assert torch.equal(a.view(torch.int16), b.view(torch.int16))
