@@ -12,9 +12,10 @@
 // 0 .. ctx - n + i).
 //
 // Head_dims and block sizes that are multiples of 8, up to head_dim 256, run
-// the matrix-core kernels of generic_decode.hip; the rest (head_dim past 256
-// or not a multiple of 8, block sizes 1, 2, 4, unaligned tensors) the scalar
-// row routine, one 256-thread workgroup per (query row, q head).
+// the matrix-core kernels of generic_decode.hip and generic_prefill.hip; the
+// rest (head_dim past 256 or not a multiple of 8, block sizes 1, 2, 4,
+// unaligned tensors, prefill of more than 128 heads a group) the scalar row
+// routine, one 256-thread workgroup per (query row, q head).
 #include "generic_attention.h"
 #include "generic_mfma.h"
 #include "workspace.h"
@@ -97,6 +98,21 @@ void gen_decode_plan(GenArgs* g, bool fp8) {
     if (units * g->parts > INT32_MAX || slots * (g->d + 2) > (int64_t(1) << 28)) g->parts = 1;
 }
 
+// Prefill: few workgroups split the keys, at most 8 parts of at least 4
+// 64-key tiles, as many as the CUs take at once (two workgroups a CU up to
+// head_dim 128, one past it).
+void gen_prefill_plan(GenArgs* g, int64_t base_wgs) {
+    const int64_t tiles = (static_cast<int64_t>(g->maxb) * g->bs + 63) / 64;
+    const int64_t want = (g->d > 128 ? 1 : 2) * int64_t(gen_cus());
+    int64_t parts = std::min<int64_t>(std::min<int64_t>(8, tiles / 4), want / base_wgs);
+    if (parts < 1) parts = 1;
+    const int64_t per = (tiles + parts - 1) / parts;
+    g->chunk = static_cast<int32_t>(per * 64);
+    g->parts = per > 0 ? static_cast<int32_t>((tiles + per - 1) / per) : 1;
+    const int64_t slots = static_cast<int64_t>(g->rows) * g->hq * g->parts;
+    if (slots * (g->d + 2) > (int64_t(1) << 28)) g->parts = 1;
+}
+
 }  // namespace
 
 int32_t generic_attention(void* out, const void* q, const void* kc, const void* vc, const int32_t* bt,
@@ -120,6 +136,15 @@ int32_t generic_attention(void* out, const void* q, const void* kc, const void* 
         if (!may_allocate) g.parts = 1;
         gen_take_scratch(&g, stream);
         return launch_gen_decode(g, q_dtype, kv_dtype, g.parts, stream);
+    }
+    if (qsl && gen_mfma_shape(g, kv_dtype) && hq / hkv <= 128) {
+        const int64_t base_wgs = gen_prefill_base_wgs(g);
+        if (base_wgs <= INT32_MAX / 8) {
+            gen_prefill_plan(&g, base_wgs);
+            if (!may_allocate) g.parts = 1;
+            gen_take_scratch(&g, stream);
+            return launch_gen_prefill(g, q_dtype, kv_dtype, base_wgs, stream);
+        }
     }
     const dim3 grid(static_cast<unsigned>(rows * hq));
     return q_dtype == KIND_BF16 ? launch_kv<KIND_BF16>(kv_dtype, g, grid, stream)

@@ -99,3 +99,64 @@ def test_decode_repeats_bitwise_and_unsplit_agrees(dev):
         torch.cuda.synchronize()
         assert_close(f32(out), f32(a), TOL_BF16, "unsplit")
     assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+# prefill: (head_dim, q heads, kv heads, block size, kind, new tokens, cached):
+# query tiles hold 128 rows (128 / G tokens), key tiles 64 keys, parts 256
+PREFILL = [
+    (96, 3, 3, 16, O.F16, [127, 128, 129, 1], [0, 0, 0, 0]),
+    (128, 6, 2, 8, O.BF16, [42, 43, 0, 85, 1], [0, 63, 5, 65, 700]),
+    (72, 5, 1, 24, O.BF16, [25, 26, 51], [0, 64, 1]),
+    (200, 34, 2, 40, O.F16, [7, 8], [600, 0]),
+    (256, 4, 4, 64, O.BF16, [129, 64], [63, 1000]),
+    (8, 128, 1, 32, O.F16, [2, 65], [30, 0]),
+]
+
+
+def _prefill_case(rng, case):
+    D, hq, hkv, bs, kind, new, cached = case
+    new, cached = np.array(new, np.int32), np.array(cached, np.int32)
+    sl = new + cached
+    _, k, v, bt, _ = random_case(rng, len(new), hq, hkv, D, (int(sl.max()), int(sl.max())), bs=bs, neg_blocks=1)
+    qsl = np.concatenate([[0], np.cumsum(new)]).astype(np.int32)
+    q = rng.standard_normal((int(qsl[-1]), hq, D)).astype(np.float32)
+    return q, k, v, bt, sl, qsl
+
+
+def _prefill(dev, kind, q, k, v, bt, sl, qsl, scale):
+    qb, kb, vb = O.encode(q, kind), O.encode(k, kind), O.encode(v, kind)
+    out = ops.paged_prefill(t16(qb, TORCH[kind], dev), t16(kb, TORCH[kind], dev), t16(vb, TORCH[kind], dev),
+                            ti(bt, torch.int32, dev), ti(sl, torch.int32, dev), ti(qsl, torch.int32, dev), scale)
+    torch.cuda.synchronize()
+    return f32(out), O.paged_attention_prefill(qb, kind, kb, vb, kind, bt, sl, qsl, scale, precision=1)
+
+
+@pytest.mark.parametrize("case", PREFILL, ids=[f"D{c[0]}-{c[1]}x{c[2]}-bs{c[3]}" for c in PREFILL])
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_prefill_edges_vs_oracle(dev, case, sign):
+    D, kind = case[0], case[4]
+    rng = np.random.default_rng(D + case[1])
+    args = _prefill_case(rng, case)
+    log_case(f"generic mfma prefill {case} sign {sign}")
+    got, ref = _prefill(dev, kind, *args, sign / np.sqrt(D))
+    assert_close(got, ref, TOL_BF16, f"prefill {case}")
+    rel = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    assert rel < 1.5 * (2.0 ** -9 if kind == O.BF16 else 2.0 ** -12), rel
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+@pytest.mark.parametrize("cached", [0, 700])   # 700: the keys are split into parts
+def test_prefill_value_that_is_not_finite_stays_in_its_rows(dev, bad, cached):
+    # the value of a new token reaches the rows that see it and no earlier one
+    case = (128, 6, 2, 16, O.BF16, [90], [cached])
+    rng = np.random.default_rng(6)
+    q, k, v, bt, sl, qsl = _prefill_case(rng, case)
+    bt[bt < 0] = np.setdiff1d(np.arange(k.shape[0]), bt)[0]   # the helper's skipped block: present here
+    pos = cached + 37
+    v[bt[0, pos // 16], 1, 3, pos % 16] = bad
+    log_case(f"generic mfma prefill value {bad} cached {cached}")
+    got, ref = _prefill(dev, O.BF16, q, k, v, bt, sl, qsl, 1 / np.sqrt(128))
+    ok = np.isfinite(ref)
+    assert ok[:37].all() and not ok[37:, 3:, 3].any()
+    assert np.array_equal(np.isfinite(got), ok) and np.array_equal(np.isposinf(got), np.isposinf(ref))
+    assert (np.abs(got[ok] - ref[ok]) <= 2e-2 + 1e-2 * np.abs(ref[ok])).all()
