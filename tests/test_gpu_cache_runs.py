@@ -1,0 +1,86 @@
+"""Cache writes of long token lists (slot runs written as whole rows) against the
+CPU oracle, bit-exact: prompts that start anywhere in the list and in a block,
+decode tokens between them, padding, blocks past the pool, and the sizes where
+groups, chunks and the choice of the kernel end."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+import rllm_amd
+from gpu_util import bits16, log_case, t16, t8, ti
+from rllm_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _slots(rng, n, bs):
+    """(slots, blocks in the pool): runs of random length at random offsets."""
+    out, nb = [], 0
+    while len(out) < n:
+        run = int(rng.choice([1, 1, 3, 15, 16, 17, 40, 200]))
+        first = int(rng.choice([0, 0, 1, 7, bs - 1]))
+        out += list(range(nb * bs + first, nb * bs + first + run))
+        nb = out[-1] // bs + 1 + int(rng.integers(0, 2))
+    out = np.array(out[:n], np.int64)
+    # blocks in any order: a run continues in an unrelated block
+    perm = rng.permutation(nb + 1)
+    out = perm[out // bs] * bs + out % bs
+    out[rng.integers(0, n, 5)] = -1
+    return out, nb - 1               # ids nb - 1 and nb lie past the pool
+
+
+# (kv heads, head_dim, block size, tokens)
+SHAPES = [(8, 128, 16, 384), (8, 128, 16, 385), (8, 128, 32, 2047), (8, 128, 16, 2049), (1, 40, 48, 700),
+          (3, 24, 16, 2500), (1, 8, 64, 399)]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=[f"{s[0]}x{s[1]}-bs{s[2]}-n{s[3]}" for s in SHAPES])
+@pytest.mark.parametrize("cache", [O.BF16, O.FP8_E4M3, O.FP8_E5M2])
+def test_cache_write_runs_bit_exact(dev, shape, cache):
+    hkv, d, bs, n = shape
+    rng = np.random.default_rng(n + d + cache)
+    sl, nb = _slots(rng, n, bs)
+    nk = O.encode(rng.standard_normal((n, hkv, d)).astype(np.float32), O.BF16)
+    nv = O.encode(rng.standard_normal((n, hkv, d)).astype(np.float32), O.BF16)
+    args = (t16(nk, torch.bfloat16, dev), t16(nv, torch.bfloat16, dev))
+    log_case(f"cache_write runs {shape} cache={cache}")
+    if cache == O.BF16:
+        kc = rng.integers(0, 65536, size=(nb, hkv, d, bs), dtype=np.uint16)
+        vc = rng.integers(0, 65536, size=(nb, hkv, d, bs), dtype=np.uint16)
+        gk, gv = t16(kc, torch.bfloat16, dev), t16(vc, torch.bfloat16, dev)
+        ops.reshape_and_cache(*args, gk, gv, ti(sl, torch.int64, dev))
+        torch.cuda.synchronize()
+        O.cache_write(kc, vc, nk, nv, sl, bs, O.BF16, O.BF16)
+        assert np.array_equal(bits16(gk), kc) and np.array_equal(bits16(gv), vc)
+        return
+    code = rllm_amd.DTYPE_FP8_E4M3 if cache == O.FP8_E4M3 else rllm_amd.DTYPE_FP8_E5M2
+    for ks, vs, rne in ((0.25, 4.0, False), (3.7 / 448.0, 0.0117, True)):
+        kc = rng.integers(0, 256, size=(nb, hkv, d, bs), dtype=np.uint8)
+        vc = rng.integers(0, 256, size=(nb, hkv, d, bs), dtype=np.uint8)
+        gk, gv = t8(kc, dev), t8(vc, dev)
+        ops.reshape_and_cache(*args, gk, gv, ti(sl, torch.int64, dev), kv_dtype=code, k_scale=ks, v_scale=vs,
+                              fp8_rounding=rllm_amd.FP8_ROUND_NEAREST_EVEN if rne
+                              else rllm_amd.FP8_ROUND_TOWARD_ZERO)
+        torch.cuda.synchronize()
+        O.cache_write(kc, vc, nk, nv, sl, bs, O.BF16, cache, ks, vs, round_nearest=rne)
+        assert np.array_equal(gk.cpu().numpy(), kc) and np.array_equal(gv.cpu().numpy(), vc)
+
+
+def test_cache_write_unaligned_rows_take_the_token_kernel(dev):
+    # rows two bytes past a 16-byte boundary: the same bytes
+    hkv, d, bs, n = 2, 64, 16, 500
+    rng = np.random.default_rng(4)
+    sl, nb = _slots(rng, n, bs)
+    nk = O.encode(rng.standard_normal((n, hkv, d)).astype(np.float32), O.F16)
+    buf = torch.empty(n * hkv * d + 1, dtype=torch.float16, device=dev)
+    x = buf[1:].view(n, hkv, d)
+    x.copy_(t16(nk, torch.float16, dev))
+    kc = np.zeros((nb, hkv, d, bs), np.uint16)
+    gk, gv = t16(kc, torch.float16, dev), t16(kc, torch.float16, dev)
+    log_case("cache_write unaligned rows")
+    ops.reshape_and_cache(x, x, gk, gv, ti(sl, torch.int64, dev))
+    torch.cuda.synchronize()
+    ek, ev = kc.copy(), kc.copy()
+    O.cache_write(ek, ev, nk, nk, sl, bs, O.F16, O.F16)
+    assert np.array_equal(bits16(gk), ek) and np.array_equal(bits16(gv), ev)
