@@ -806,7 +806,7 @@ __global__ __launch_bounds__(PP_THREADS, 1) void cascade_kernel(PrefillArgs pa, 
     __shared__ uint4 lds[WORDS];
     const int b = static_cast<int>(blockIdx.x);
     if (b < prefix_wgs) {
-        prefill_body<QKIND, KVKIND, D, G>(pa, block_tables, b, lds);
+        prefill_body<QKIND, KVKIND, D, G, true>(pa, block_tables, b, lds);
         return;
     }
     const int wid = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -1332,7 +1332,7 @@ __global__ __launch_bounds__(PP_THREADS, 1) void mixed_kernel(PrefillArgs pa, co
     __shared__ uint4 lds[WORDS];
     const int b = static_cast<int>(blockIdx.x);
     if (b < prefill_wgs) {
-        prefill_body<QKIND, KVKIND, D, G>(pa, block_tables, b, lds);
+        prefill_body<QKIND, KVKIND, D, G, false>(pa, block_tables, b, lds);
         return;
     }
     const int wid = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -1741,7 +1741,9 @@ int32_t decode_prefix_impl(void* out, const void* q, const void* kc, const void*
     Kernels kern;
     RLLM_CHECK_ARG(pick_kernels(q_dtype, kv_dtype, d, G, &kern));
 
-    const int64_t S = prefix_partial_splits(num_seqs, hq, hkv, prefix_blocks);
+    const bool fp8_kv = kv_dtype == KIND_FP8_E4M3 || kv_dtype == KIND_FP8_E5M2;
+    const int64_t S = prefix_partial_splits(num_seqs, hq, hkv, d, prefix_blocks,
+                                            num_seqs * hkv * (maxb - prefix_blocks) * bs * d * (fp8_kv ? 2 : 4));
     // the suffix partitions: whole 512-token chunks, as few per partition as
     // keep the widest suffix within CASCADE_MAX_SUFFIX_PARTS partitions
     const int64_t rest_chunks = (maxb - prefix_blocks + SC_BLOCKS - 1) / SC_BLOCKS;

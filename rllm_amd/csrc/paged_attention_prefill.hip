@@ -21,7 +21,7 @@ template <int QKIND, int KVKIND, int D, int G>
 __global__ __launch_bounds__(PP_THREADS, 1) void prefill_kernel(PrefillArgs a,
                                                                 const int32_t* __restrict__ block_tables) {
     __shared__ uint4 lds[pf_lds_words<D>()];
-    prefill_body<QKIND, KVKIND, D, G>(a, block_tables, static_cast<int>(blockIdx.x), lds);
+    prefill_body<QKIND, KVKIND, D, G, false>(a, block_tables, static_cast<int>(blockIdx.x), lds);
 }
 
 // Merges the KV splits of every output row (token * Hq + q head): one wave
@@ -194,6 +194,11 @@ int32_t prefill_impl(void* out, const void* q, const void* kc, const void* vc, c
     const int64_t splits = chunk_splits(nwg, maxb);
     a.splits = static_cast<int32_t>(splits);
     a.base_wgs = static_cast<int32_t>(nwg);
+    // more workgroups than CUs: the longest tiles first (5 prompts of 1459 fresh
+    // tokens, 16/4 heads: 74.6 us sequence by sequence, 58.2 so; 8 of 512 on
+    // 2048: 147.7, 143.9; 6 of 237-1541: 83.6, 86.6).  A single round keeps the
+    // cheaper lookup.
+    a.longest_first = splits == 1 && nwg > device_cu_count() && num_seqs <= LONGEST_MAX_SEQS;
     const int64_t rows = num_tokens * hq;
     int64_t splits_used = splits;
     if (splits > 1) {
@@ -260,12 +265,27 @@ int32_t sync_after(int32_t rc) {
 // cascade runs that mode inside its own kernel (cascade_kernel,
 // paged_attention_decode.hip); these helpers size it.
 
-// The prefill rule (a split keeps at least 4 of the prefix's 64-token tiles):
-// the partials run beside the suffix decode, so fewer, longer workgroups
-// leave it more CUs; 2-tile splits measured no faster (20.1 -> 21.0 us on
-// config 4a) and cost the reduction a partial more per row.
-int64_t prefix_partial_splits(int64_t num_seqs, int64_t hq, int64_t hkv, int64_t prefix_blocks) {
-    return prefill_splits(prefix_base_wgs(num_seqs, hq, hkv), prefix_blocks);
+// The partials run beside the suffix decode, so fewer, longer workgroups leave
+// it more CUs and the reduction fewer partials: the fewest splits whose
+// workgroups (about PREFIX_WG_NS and PREFIX_TILE_NS a 64-key tile) still end
+// within 85% of the time the suffix's bytes take (about SUFFIX_GBPS; its
+// length is the table's, an upper bound).  Where none does, the prefix is what
+// the call waits for: the prefill rule (a split keeps at least 4 tiles).  32/8
+// heads, D 128, us with 1 / 2 / 3 splits / the prefill rule's: 128 sequences
+// on 64 + 16 blocks 37.7 / 32.9 / 33.6 / 33.9 (4), 128 on 128 + 16 57.0 / 38.9
+// / 34.4 / 41.4 (8), 64 on 64 + 16 35.0 / 26.1 / 23.6 / 21.5 (4).
+constexpr int64_t PREFIX_WG_NS = 7500, PREFIX_TILE_NS = 1750, PREFIX_TILE_NS_64 = 1200, SUFFIX_GBPS = 5000;
+
+int64_t prefix_partial_splits(int64_t num_seqs, int64_t hq, int64_t hkv, int64_t d, int64_t prefix_blocks,
+                              int64_t suffix_bytes) {
+    const int64_t most = prefill_splits(prefix_base_wgs(num_seqs, hq, hkv), prefix_blocks);
+    const int64_t tiles = (prefix_blocks + PF_NBT - 1) / PF_NBT;
+    const int64_t suffix_ns = suffix_bytes / SUFFIX_GBPS;
+    for (int64_t sp = 1; sp < most; ++sp) {
+        const int64_t ns = PREFIX_WG_NS + (d == 64 ? PREFIX_TILE_NS_64 : PREFIX_TILE_NS) * ((tiles + sp - 1) / sp);
+        if (ns * 20 <= suffix_ns * 17) return sp;
+    }
+    return most;
 }
 
 bool prefix_partials_supported(int64_t hq, int64_t hkv, int64_t d, int64_t bs, int32_t q_dtype, int32_t kv_dtype,

@@ -14,8 +14,9 @@
 //               G = Hq/Hkv heads of the GQA group x 256/G query tokens, so
 //               every K/V tile staged in LDS serves the whole group.  One
 //               workgroup per CU, two waves per SIMD.  A sequence's last
-//               query tile (the most keys) is launched first, so the
-//               workgroups that start later are the short ones.
+//               query tile (the most keys) is launched first, or, in a
+//               grid of several rounds, the batch's tiles by falling key
+//               counts, so the workgroups that start later are the short ones.
 //   KV tile   = 64 tokens (four cache blocks) in LDS in the cache's own
 //               layout ([block][d][16 tokens]), three buffers.
 //   ping-pong = waves 0-3 (group 0) and 4-7 (group 1) take turns: while one
@@ -132,7 +133,12 @@ struct PrefillArgs {
     // block_tables[0] (max_blocks = the prefix's blocks), and every row of
     // the batch writes a partial, also with one split
     int32_t prefix_tokens, prefix_queries;
+    // query tiles in the order of falling key counts over all sequences
+    // (longest_tile) instead of sequence by sequence; at most LONGEST_MAX_SEQS
+    int32_t longest_first;
 };
+
+constexpr int LONGEST_MAX_SEQS = 16;
 
 // Transposing LDS read: in each group of 16 lanes, lane j addresses 4
 // consecutive 16-bit values M[j][0..3]; lane i receives M[4k + i/4][i%4]
@@ -210,6 +216,48 @@ __device__ __forceinline__ uint4 cvt8(uint2 a) {
     return make_uint4(d[0], d[1], d[2], d[3]);
 }
 
+// inclusive prefix sum over the wave (DPP)
+__device__ __forceinline__ int seq_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);   // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);   // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);   // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);   // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);   // row_bcast:15 into rows 1, 3
+    return v + __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);   // row_bcast:31 into rows 2, 3
+}
+
+// Tile `rank` of the batch in the order of falling key counts, in 64 steps of
+// 64 keys (wider past 4096; equal steps by sequence): the sequence and its
+// tile, -1 past the last tile that sees a key.  The workgroups of a launch
+// start in order, so the longest run first and the short ones fill the last
+// round.  Lane i brings sequence i's new tokens n and context ctx; the answer
+// is uniform.
+template <int QT>
+__device__ __forceinline__ int longest_tile(int num_seqs, int lane, int n, int ctx, int rank, int& tile) {
+    static_assert((QT & (QT - 1)) == 0, "tiles are counted by shifts");
+    constexpr int SH = __builtin_ctz(QT);
+    // tiles of a sequence with more than thr keys: its last ones (tile i sees
+    // ctx - n + min((i + 1) QT, n) keys)
+    auto above = [](int n, int ctx, int thr) {
+        return n > 0 && ctx > thr ? ((n + QT - 1) >> SH) - max(0, (thr - (ctx - n)) >> SH) : 0;
+    };
+    int widest = 0;
+    for (int s = 0; s < num_seqs; ++s) widest = max(widest, __builtin_amdgcn_readlane(ctx, s));
+    const int step = PF_KT * max(1, (widest + 64 * PF_KT - 1) / (64 * PF_KT));
+    int count = 0;                          // tiles past this lane's threshold
+    for (int s = 0; s < num_seqs; ++s)
+        count += above(__builtin_amdgcn_readlane(n, s), __builtin_amdgcn_readlane(ctx, s), lane * step);
+    const int u = __popcll(__builtin_amdgcn_ballot_w64(count > rank)) - 1;   // counts fall with the lane
+    if (u < 0) return -1;
+    const int r = rank - (u < 63 ? __builtin_amdgcn_readlane(count, min(u + 1, 63)) : 0);
+    const int top = above(n, ctx, (u + 1) * step), band = above(n, ctx, u * step) - top;   // tiles in this step
+    const int before = seq_scan(band) - band;
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(before <= r && r < before + band);
+    const int s = __ffsll(static_cast<unsigned long long>(hit)) - 1;
+    tile = __builtin_amdgcn_readlane(((n + QT - 1) >> SH) - top - 1 - (r - before), s);
+    return s;
+}
+
 // LDS of the kernel body: PP_NBUF K and PP_NBUF V tile buffers, in 16-byte
 // words
 template <int D>
@@ -224,7 +272,8 @@ constexpr int pf_lds_words() {
 // struct made the compiler copy part of it into LDS, thread by thread, which
 // reads the dispatch packet in every wave and slowed the launch of the
 // workgroups to about one every 50 ns across the device.
-template <int QKIND, int KVKIND, int D, int G>
+// PREFIX: the shared-prefix mode (a.prefix_tokens > 0), else the chunked one.
+template <int QKIND, int KVKIND, int D, int G, bool PREFIX>
 __device__ __forceinline__ void prefill_body(PrefillArgs a, const int32_t* __restrict__ block_tables, const int bid,
                                              uint4* lds) {
     using M = Mfma<QKIND>;
@@ -255,11 +304,35 @@ __device__ __forceinline__ void prefill_body(PrefillArgs a, const int32_t* __res
     const int split = a.splits > 1 ? bid / a.base_wgs : 0;
     const int h = base % a.num_kv_heads;
     int j = base / a.num_kv_heads;
-    const bool prefix_mode = a.prefix_tokens > 0;
-    int s = 0, n = 0, q0 = 0;
-    if (prefix_mode) {
+    int s = 0, n = 0, q0 = 0, ctx = 0, tile;
+    if constexpr (PREFIX) {
         n = a.prefix_queries;
-        if (j >= (n + QT - 1) / QT) return;   // whole workgroup
+        tile = (n + QT - 1) / QT - 1 - j;
+        if (tile < 0) return;                 // whole workgroup
+        ctx = a.prefix_tokens;
+    } else if (a.num_seqs <= 64) {
+        // lane i holds sequence i
+        int q0_l = 0, n_l = 0, ctx_l = 0;
+        if (lane < a.num_seqs) {
+            q0_l = a.query_start_loc[lane];
+            n_l = a.query_start_loc[lane + 1] - q0_l;
+            ctx_l = a.seq_lens[lane];
+        }
+        if (a.longest_first) {
+            s = longest_tile<QT>(a.num_seqs, lane, n_l, ctx_l, j, tile);
+            if (s < 0) return;                // whole workgroup: no barrier is reached
+        } else {
+            const int nt_l = n_l > 0 ? (n_l + QT - 1) / QT : 0;
+            const int first_l = seq_scan(nt_l) - nt_l;
+            const uint64_t hit = __builtin_amdgcn_ballot_w64(first_l <= j && j < first_l + nt_l);
+            if (!hit) return;                 // whole workgroup
+            s = __ffsll(static_cast<unsigned long long>(hit)) - 1;
+            // a sequence's last query tile (the most keys) first
+            tile = __builtin_amdgcn_readlane(nt_l - 1 - (j - first_l), s);
+        }
+        q0 = __builtin_amdgcn_readlane(q0_l, s);
+        n = __builtin_amdgcn_readlane(n_l, s);
+        ctx = __builtin_amdgcn_readlane(ctx_l, s);
     } else {
         for (; s < a.num_seqs; ++s) {
             q0 = a.query_start_loc[s];
@@ -268,14 +341,14 @@ __device__ __forceinline__ void prefill_body(PrefillArgs a, const int32_t* __res
             if (j < nt) break;
             j -= nt;
         }
-        if (s >= a.num_seqs) return;      // whole workgroup: no barrier is reached
+        if (s >= a.num_seqs) return;          // whole workgroup
+        ctx = a.seq_lens[s];
+        tile = (n + QT - 1) / QT - 1 - j;
     }
-    j = (n + QT - 1) / QT - 1 - j;    // the sequence's last query tile first
-    const int qt0 = j * QT;
-    const int ctx = prefix_mode ? a.prefix_tokens : a.seq_lens[s];
+    const int qt0 = tile * QT;
     const int cached = ctx - n;
     const int last_q = min(qt0 + QT, n) - 1;
-    const int kv_end = prefix_mode ? min(ctx, a.max_blocks * PF_BS)
+    const int kv_end = PREFIX ? min(ctx, a.max_blocks * PF_BS)
                                    : min(min(cached + last_q + 1, ctx), a.max_blocks * PF_BS);
     const int ntiles = kv_end > 0 ? (kv_end + PF_KT - 1) / PF_KT : 0;
     const int per_split = (ntiles + a.splits - 1) / a.splits;
@@ -323,31 +396,44 @@ __device__ __forceinline__ void prefill_body(PrefillArgs a, const int32_t* __res
         return ((1 << nin) - 1) & ~neg;
     };
 
+    vec qreg[NKS];    // B operand of k-step k: Q[row][16k + 8hl .. +7]
+    // Q scaled once by scale * log2(e) (rounded to the q type), so the products
+    // give scores in log2 units
+    auto scale_q = [&]() __attribute__((always_inline)) -> void {
+#pragma unroll
+        for (int k = 0; k < NKS; ++k) {
+            f32x8 y = __builtin_convertvector(qreg[k], f32x8) * a.s_scale;
+            qreg[k] = __builtin_convertvector(y, typename M::elem8);
+        }
+    };
     // ---- this lane's query row: m = 32 * wave + l32 -> (head g, token i) ----
     int pos;          // absolute position of the row's query token (-1: no row)
     int64_t orow;     // output row index (token * Hq + q head)
     bool row_out;     // the row has an output (a partial, in the shared-prefix mode)
-    vec qreg[NKS];    // B operand of k-step k: Q[row][16k + 8hl .. +7]
     {
         const int m = 32 * wave + l32;
         const int g = m / QT, i = qt0 + m % QT;
         const bool live = i < n;
         // shared-prefix mode: the last key the row attends (-1: none, a
         // sequence with no context; its partial is then empty)
-        pos = !live ? -1 : prefix_mode ? min(max(a.seq_lens[i], 0), ctx) - 1 : cached + i;
-        row_out = prefix_mode ? live : pos >= 0;
+        pos = !live ? -1 : PREFIX ? min(max(a.seq_lens[i], 0), ctx) - 1 : cached + i;
+        row_out = PREFIX ? live : pos >= 0;
         orow = (static_cast<int64_t>(q0) + i) * a.num_q_heads + h * G + g;
+        // read here, scaled (scale_q) once the first copies are under way; rows
+        // without a query read the tile's first
+        const uint16_t* qsrc = a.q + (live ? orow : (static_cast<int64_t>(q0) + qt0) * a.num_q_heads + h * G) * D;
 #pragma unroll
         for (int k = 0; k < NKS; ++k) {
             uint4 w = make_uint4(0, 0, 0, 0);
-            if (live) w = *reinterpret_cast<const uint4*>(a.q + orow * D + 16 * k + 8 * hl);
-            // Q scaled once by scale * log2(e) (rounded to the q type), so the
-            // products give scores in log2 units
-            vec x = __builtin_bit_cast(vec, w);
-            f32x8 y = __builtin_convertvector(x, f32x8) * a.s_scale;
-            qreg[k] = __builtin_convertvector(y, typename M::elem8);
+            if (!PREFIX || live) w = *reinterpret_cast<const uint4*>(qsrc + 16 * k + 8 * hl);
+            qreg[k] = __builtin_bit_cast(vec, w);
         }
+        // beside the suffix waves, at once: 33.8 -> 33.4 us for 128 sequences on
+        // a 64-block prefix with 16 blocks each
+        if constexpr (PREFIX) scale_q();
     }
+    // rows without an output never hold a tile back from the fast softmax
+    const uint64_t out_rows = __builtin_amdgcn_ballot_w64(row_out);
     // smallest position among the wave's rows: tiles wholly at or below it
     // need no causal mask for any row of the wave
     // (a shared-prefix row that attends nothing counts: its keys are masked)
@@ -420,10 +506,6 @@ __device__ __forceinline__ void prefill_body(PrefillArgs a, const int32_t* __res
     for (int dt = 0; dt < NDT; ++dt) o[dt] = f32x16{};
     f32x16 st[2];                 // S^T of the tile's 32-token halves
     uint32_t pk[2][8];            // 16-bit weights, packed pairs, same order
-#pragma unroll
-    for (int sh = 0; sh < 2; ++sh)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) pk[sh][e] = 0;
     float m_run = -INFINITY, l_run = 0.f;   // m in scaled log2 units; l: this lane's share of the row sum
 
     // ---- matrix phase ----
@@ -452,8 +534,9 @@ __device__ __forceinline__ void prefill_body(PrefillArgs a, const int32_t* __res
     // t.  Operands are read one step ahead (register rings), so every
     // product's LDS reads were issued a step of products earlier;
     // sched_barrier keeps the compiler's scheduler from moving each read next
-    // to its product to save registers.
-    auto mphase = [&](int bc) __attribute__((always_inline)) -> void {
+    // to its product to save registers.  The workgroup's first tile (`first`, a
+    // literal at every call) has no V before it.
+    auto mphase = [&](int bc, bool first) __attribute__((always_inline)) -> void {
         vec vop[2][NDT];
         vec kop[2][2];
         auto load_v = [&](int b, vec* dst) __attribute__((always_inline)) {
@@ -468,15 +551,19 @@ __device__ __forceinline__ void prefill_body(PrefillArgs a, const int32_t* __res
                 dst[sh] = __builtin_bit_cast(vec, __builtin_shufflevector(k0, k1, 0, 1, 2, 3, 4, 5, 6, 7));
             }
         };
-        load_v(0, vop[0]);
+        if (first) {
+            load_k(0, kop[0]);
+        } else {
+            load_v(0, vop[0]);
 #pragma unroll
-        for (int b = 0; b < PF_NBT; ++b) {
-            if (b + 1 < PF_NBT) load_v(b + 1, vop[(b + 1) & 1]);
-            else load_k(0, kop[0]);
-            __builtin_amdgcn_sched_barrier(0);
-            const vec pb = pv_b(b);
+            for (int b = 0; b < PF_NBT; ++b) {
+                if (b + 1 < PF_NBT) load_v(b + 1, vop[(b + 1) & 1]);
+                else load_k(0, kop[0]);
+                __builtin_amdgcn_sched_barrier(0);
+                const vec pb = pv_b(b);
 #pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) o[dt] = M::mma(vop[b & 1][dt], pb, o[dt]);
+                for (int dt = 0; dt < NDT; ++dt) o[dt] = M::mma(vop[b & 1][dt], pb, o[dt]);
+            }
         }
         // S^T starts at -m_run (0 while a row has no max yet): the fast
         // softmax then takes exp2 of the product directly
@@ -537,7 +624,7 @@ __device__ __forceinline__ void prefill_body(PrefillArgs a, const int32_t* __res
     auto softmax_fast = [&](int t, int pres) __attribute__((always_inline)) -> bool {
         const int t_base = t * PF_KT;
         const bool full = pres == (1 << PF_NBT) - 1 && t_base + PF_KT <= kv_end && t_base + PF_KT - 1 <= minp;
-        if (!full || __builtin_amdgcn_ballot_w64(m_run == -INFINITY)) return false;
+        if (!full || (__builtin_amdgcn_ballot_w64(m_run == -INFINITY) & out_rows)) return false;
         float acc_a = 0.f, acc_b = 0.f;
 #pragma unroll
         for (int sh = 0; sh < 2; ++sh)
@@ -551,7 +638,7 @@ __device__ __forceinline__ void prefill_body(PrefillArgs a, const int32_t* __res
                 acc_b += p1;
             }
         const float acc_s = acc_a + acc_b;
-        if (__builtin_amdgcn_ballot_w64(!(acc_s <= 256.f))) return false;
+        if (__builtin_amdgcn_ballot_w64(!(acc_s <= 256.f)) & out_rows) return false;
         l_run += acc_s;
         return true;
     };
@@ -626,8 +713,7 @@ __device__ __forceinline__ void prefill_body(PrefillArgs a, const int32_t* __res
         load_entries(t_lo);
         int pres = presence(t_lo);
         // prologue: K_{t_lo} into buffer 0, K_{t_lo+1} and V_{t_lo} into
-        // buffer 1; zeros as V of buffer 0 (the first tile's products add
-        // zero weights times zeros, so every tile runs the same code)
+        // buffer 1
         if (grp == 0) {
             fetch(true, entry(t_lo, my_blk), 0);
             if constexpr (FP8) {
@@ -641,13 +727,9 @@ __device__ __forceinline__ void prefill_body(PrefillArgs a, const int32_t* __res
                 stage(true, 1);
                 stage(false, 1);
             }
-        } else {
-            uint4* vz = reinterpret_cast<uint4*>(&v_lds[0][0][0][0]);
-            constexpr int NZ = static_cast<int>(sizeof(TileBuf) / sizeof(uint4));
-#pragma unroll
-            for (int i = tid - 256; i < NZ; i += 256) vz[i] = make_uint4(0, 0, 0, 0);
         }
         load_entries(t_lo + 1);   // tile t_lo + 1 (and K of t_lo + 2) for the first copies
+        if constexpr (!PREFIX) scale_q();
         __builtin_amdgcn_s_waitcnt(0);
         __builtin_amdgcn_s_barrier();
         if (grp == 1) __builtin_amdgcn_s_barrier();
@@ -660,8 +742,8 @@ __device__ __forceinline__ void prefill_body(PrefillArgs a, const int32_t* __res
         // earlier.  Issued as the softmax phase starts, the copies overlap its
         // arithmetic and have three phases to land; the entries of the next
         // pair start to load.
-        auto tile_front = [&](int t, int bc) __attribute__((always_inline)) -> void {
-            mphase(bc);
+        auto tile_front = [&](int t, int bc, bool first) __attribute__((always_inline)) -> void {
+            mphase(bc, first);
             __builtin_amdgcn_s_barrier();
             const int b1 = bc == PP_NBUF - 1 ? 0 : bc + 1;   // buffer of tile t + 1
             const int b2 = bc == 0 ? PP_NBUF - 1 : bc - 1;   // buffer of tile t + 2
@@ -692,12 +774,15 @@ __device__ __forceinline__ void prefill_body(PrefillArgs a, const int32_t* __res
         // resumes (a rescale inside the loop body makes the register
         // allocator copy the accumulators between two register sets on
         // every tile).
-        int t = t_lo, bcur = 0;   // bcur: buffer of tile t
         auto next_buf = [](int b) { return b == PP_NBUF - 1 ? 0 : b + 1; };
+        tile_front(t_lo, 0, true);
+        softmax_exact(t_lo, pres);   // no running max yet
+        tile_back(t_lo);
+        int t = t_lo + 1, bcur = 1;   // bcur: buffer of tile t
         while (t < t_hi) {
             bool exact = false;
             for (; t < t_hi; ++t, bcur = next_buf(bcur)) {
-                tile_front(t, bcur);
+                tile_front(t, bcur, false);
                 if (!softmax_fast(t, pres)) {
                     exact = true;
                     break;
@@ -721,8 +806,8 @@ __device__ __forceinline__ void prefill_body(PrefillArgs a, const int32_t* __res
 
     // ---- normalise and store: lane holds out[row][32dt + 8jj + 4hl + 0..3] ----
     const float l = xor_sum_32(l_run);
-    if (!row_out) return;
-    if (a.splits > 1 || prefix_mode) {   // this split's normalised partial and (max, sum) of the row
+    if (!row_out) return;   // lanes l and l + 32 hold one row: they leave together
+    if (PREFIX || a.splits > 1) {   // this split's normalised partial and (max, sum) of the row
         const float pinv = l > 0.f ? 1.f / l : 0.f;
         const int64_t slot = orow * a.part_stride + a.part_base + split;
         float* po = a.part_o + slot * D;
@@ -740,17 +825,25 @@ __device__ __forceinline__ void prefill_body(PrefillArgs a, const int32_t* __res
         }
         return;
     }
+    // lanes l and l + 32 hold the two halves of each 16-byte run; swapped in
+    // pairs of runs, lane l stores the whole run 2r and lane l + 32 run 2r + 1
     const float inv = l > 0.f ? a.v_scale / l : 0.f;
-    uint16_t* dst = static_cast<uint16_t*>(a.out) + orow * D;
+    uint16_t* dst = static_cast<uint16_t*>(a.out) + orow * D + 8 * hl;
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
+        for (int jj = 0; jj < 4; jj += 2) {
             const f32x16 x = o[dt];
-            uint2 w;
-            w.x = M::pack2(x[4 * jj] * inv, x[4 * jj + 1] * inv);
-            w.y = M::pack2(x[4 * jj + 2] * inv, x[4 * jj + 3] * inv);
-            *reinterpret_cast<uint2*>(dst + 32 * dt + 8 * jj + 4 * hl) = w;
+            uint32_t w[4];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const uint32_t even = M::pack2(x[4 * jj + 2 * i] * inv, x[4 * jj + 2 * i + 1] * inv);
+                const uint32_t odd = M::pack2(x[4 * jj + 4 + 2 * i] * inv, x[4 * jj + 5 + 2 * i] * inv);
+                const auto r = __builtin_amdgcn_permlane32_swap(even, odd, false, false);
+                w[i] = r[0];
+                w[2 + i] = r[1];
+            }
+            *reinterpret_cast<uint4*>(dst + 32 * dt + 8 * jj) = make_uint4(w[0], w[1], w[2], w[3]);
         }
 }
 
