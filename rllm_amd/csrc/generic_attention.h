@@ -17,6 +17,14 @@ int32_t generic_attention(void* out, const void* q, const void* kc, const void* 
                           int32_t q_dtype, int32_t kv_dtype, float k_scale, float v_scale, bool may_allocate,
                           hipStream_t stream);
 
+// Decode of a specialised shape (block size 16) on the shape-general kernels,
+// where they are the faster: false when the call is not taken (nothing was
+// launched), else *rc is its result.
+bool general_decode(void* out, const void* q, const void* kc, const void* vc, const int32_t* bt,
+                    const int32_t* seq_lens, int64_t num_seqs, int64_t hq, int64_t hkv, int64_t d, int64_t maxb,
+                    float scale, int32_t q_dtype, int32_t kv_dtype, float k_scale, float v_scale, hipStream_t stream,
+                    int32_t* rc);
+
 // head_dim 64 / 128, block size 16 and GQA 1, 2, 4, 8 have specialised kernels
 inline bool specialised_shape(int64_t hq, int64_t hkv, int64_t d, int64_t bs) {
     const int64_t g = hq / hkv;

@@ -1576,6 +1576,13 @@ int32_t decode_impl(void* out, const void* q, const void* kc, const void* vc, co
     if (!specialised_shape(hq, hkv, d, bs))
         return generic_attention(out, q, kc, vc, bt, seq_lens, nullptr, num_seqs, num_seqs, hq, hkv, d, bs, maxb,
                                  scale, q_dtype, kv_dtype, k_scale, v_scale, !fixed_scratch, as_stream(stream));
+    // automatic plan without a caller's workspace: short tables and few rows
+    // may run the shape-general kernels
+    int32_t general_rc = 0;
+    if (partition_size == 0 && !workspace && !fixed_scratch &&
+        general_decode(out, q, kc, vc, bt, seq_lens, num_seqs, hq, hkv, d, maxb, scale, q_dtype, kv_dtype, k_scale,
+                       v_scale, as_stream(stream), &general_rc))
+        return general_rc;
     Kernels kern;
     RLLM_CHECK_ARG(pick_kernels(q_dtype, kv_dtype, d, G, &kern));
 

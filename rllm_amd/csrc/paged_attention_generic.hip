@@ -62,10 +62,10 @@ int gen_cus() {
     return cus;
 }
 
-// Scratch of a split call, or parts = 1 where there is none to be had (a
-// capture on a stream without it, no memory left): the call then runs unsplit.
-void gen_take_scratch(GenArgs* g, hipStream_t stream) {
-    if (g->parts <= 1) return;
+// Scratch of a split call; false and parts = 1 where there is none to be had (a
+// capture on a stream without it, no memory left).
+bool gen_take_scratch(GenArgs* g, hipStream_t stream) {
+    if (g->parts <= 1) return true;
     const int64_t slots = static_cast<int64_t>(g->rows) * g->hq * g->parts;
     void* ws = nullptr;
     const int32_t rc = g_workspaces.get(reinterpret_cast<uintptr_t>(stream), WS_GENERIC, slots * (g->d + 2) * 4, false,
@@ -73,10 +73,11 @@ void gen_take_scratch(GenArgs* g, hipStream_t stream) {
     if (rc) (void)hipGetLastError();
     if (rc || !ws) {
         g->parts = 1;
-        return;
+        return false;
     }
     g->part_o = static_cast<float*>(ws);
     g->part_ml = g->part_o + slots * g->d;
+    return true;
 }
 
 // Decode: parts of whole 512-token rounds (one window for each of a
@@ -113,7 +114,58 @@ void gen_prefill_plan(GenArgs* g, int64_t base_wgs) {
     if (slots * (g->d + 2) > (int64_t(1) << 28)) g->parts = 1;
 }
 
+GenArgs gen_args(void* out, const void* q, const void* kc, const void* vc, const int32_t* bt, const int32_t* seq_lens,
+                 const int32_t* qsl, int64_t num_seqs, int64_t rows, int64_t hq, int64_t hkv, int64_t d, int64_t bs,
+                 int64_t maxb, float scale, bool fp8, float k_scale, float v_scale) {
+    return GenArgs{out, static_cast<const uint16_t*>(q), kc, vc, bt, seq_lens, qsl, static_cast<int32_t>(num_seqs),
+                   static_cast<int32_t>(hq), static_cast<int32_t>(hkv), static_cast<int32_t>(d),
+                   static_cast<int32_t>(bs), static_cast<int32_t>(maxb),
+                   scale * 1.4426950408889634f * (fp8 ? k_scale : 1.f), fp8 ? v_scale : 1.f,
+                   static_cast<int32_t>(rows), 0, 1, nullptr, nullptr};
+}
+
+// Where the general decode beats the stream decode on the stream's own shapes
+// (block size 16, G = 1, 2, 4, 8): few rows, so that four waves a row and part
+// still leave CUs free, and
+//   - tables below 8 blocks, where a stream wave walks several rows in turn
+//     (a 4-block table is an even split and stays with it for G <= 2);
+//   - G = 8, whose stream waves carry 8 heads of vector work: up to 512 tokens,
+//     or long contexts;
+//   - G = 4: one 512-token part a row, or long contexts of few rows, which the
+//     stream cuts into at most one wave a 32 blocks.
+// Kernel us, stream / general, bf16, head_dim 128, sequences x tokens: G = 4
+// (32/8 heads) 8 x 32 19.8 / 8.7, 64 x 512 27.5 / 24.3, 1 x 16384 49.6 / 22.3, 4
+// x 8192 32.3 / 29.2; kept: 8 x 512 11.8 / 13.7, 64 x 1024 46.0 / 51.2, 8 x 4096
+// 28.4 / 29.0.  G = 8 (32/4) 8 x 64 18.7 / 9.1, 8 x 512 15.8 / 13.5, 1 x 32768
+// 99.8 / 25.2, 16 x 4096 32.6 / 29.1; E4M3, head_dim 64: kept 64 x 4096 41.7 /
+// 49.3.  G = 2 (16/8) 8 x 32 14.5 / 8.6; kept 8 x 256 9.4 / 11.5.  G = 1 (8/8) 8 x
+// 32 11.8 / 8.6; kept 8 x 64 8.0 / 9.2.
+bool general_decode_pays(int64_t units, int64_t g, int64_t maxb) {
+    if (units > 512) return false;
+    if (maxb < 8) return g >= 4 || maxb <= 2 || (g == 2 && maxb != 4);
+    const int64_t tokens = maxb * 16;
+    const bool few = units * tokens <= 262144;
+    if (g >= 8) return tokens <= 512 || (tokens >= 4096 && few);
+    if (g == 4) return (tokens > 256 && tokens <= 512 && units >= 256) || (tokens >= 8192 && few);
+    return false;
+}
+
 }  // namespace
+
+bool general_decode(void* out, const void* q, const void* kc, const void* vc, const int32_t* bt,
+                    const int32_t* seq_lens, int64_t num_seqs, int64_t hq, int64_t hkv, int64_t d, int64_t maxb,
+                    float scale, int32_t q_dtype, int32_t kv_dtype, float k_scale, float v_scale, hipStream_t stream,
+                    int32_t* rc) {
+    if (!general_decode_pays(num_seqs * hkv, hq / hkv, maxb)) return false;
+    const bool fp8 = kv_dtype == KIND_FP8_E4M3 || kv_dtype == KIND_FP8_E5M2;
+    GenArgs g = gen_args(out, q, kc, vc, bt, seq_lens, nullptr, num_seqs, num_seqs, hq, hkv, d, 16, maxb, scale, fp8,
+                         k_scale, v_scale);
+    if (!gen_mfma_shape(g, kv_dtype)) return false;
+    gen_decode_plan(&g, fp8);
+    if (!gen_take_scratch(&g, stream)) return false;
+    *rc = launch_gen_decode(g, q_dtype, kv_dtype, g.parts, stream);
+    return true;
+}
 
 int32_t generic_attention(void* out, const void* q, const void* kc, const void* vc, const int32_t* bt,
                           const int32_t* seq_lens, const int32_t* qsl, int64_t num_seqs, int64_t rows,
@@ -126,10 +178,8 @@ int32_t generic_attention(void* out, const void* q, const void* kc, const void* 
     RLLM_CHECK_ARG(rows * hq <= (int64_t(1) << 31) - 1);
     if (rows <= 0) return 0;
     const bool fp8 = kv_dtype == KIND_FP8_E4M3 || kv_dtype == KIND_FP8_E5M2;
-    GenArgs g{out, static_cast<const uint16_t*>(q), kc, vc, bt, seq_lens, qsl, static_cast<int32_t>(num_seqs),
-              static_cast<int32_t>(hq), static_cast<int32_t>(hkv), static_cast<int32_t>(d), static_cast<int32_t>(bs),
-              static_cast<int32_t>(maxb), scale * 1.4426950408889634f * (fp8 ? k_scale : 1.f), fp8 ? v_scale : 1.f,
-              static_cast<int32_t>(rows), 0, 1, nullptr, nullptr};
+    GenArgs g = gen_args(out, q, kc, vc, bt, seq_lens, qsl, num_seqs, rows, hq, hkv, d, bs, maxb, scale, fp8, k_scale,
+                         v_scale);
     const int64_t units = num_seqs * hkv * ((hq / hkv + 15) / 16);
     if (!qsl && gen_mfma_shape(g, kv_dtype) && units <= INT32_MAX) {
         gen_decode_plan(&g, fp8);

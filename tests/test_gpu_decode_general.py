@@ -1,0 +1,58 @@
+"""Decode of the stream kernel's own shapes where short tables or few rows run
+the shape-general kernels instead: both sides of every line of the rule, against
+the oracle and the stream (an explicit workspace always takes it)."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+import rllm_amd
+from gpu_util import f32, log_case, t16, t8, ti
+from helpers import TOL_BF16, TOL_FP8, assert_close, random_case
+from rllm_amd import ops
+from rllm_amd.attention import decode_workspace_size
+
+pytestmark = pytest.mark.gpu
+
+# (sequences, q heads, kv heads, head_dim, table blocks, cache)
+CASES = [(5, 8, 8, 64, 2, O.BF16), (5, 8, 8, 64, 3, O.BF16), (3, 16, 8, 128, 7, O.BF16), (3, 16, 8, 128, 8, O.BF16),
+         (64, 32, 8, 128, 2, O.BF16), (65, 32, 8, 128, 2, O.BF16), (32, 32, 8, 64, 17, O.FP8_E4M3),
+         (32, 32, 8, 64, 16, O.FP8_E4M3), (32, 32, 8, 128, 33, O.BF16), (1, 4, 1, 128, 512, O.BF16),
+         (1, 4, 1, 128, 511, O.BF16), (2, 32, 4, 64, 32, O.FP8_E5M2), (2, 32, 4, 64, 33, O.BF16),
+         (2, 8, 1, 128, 256, O.BF16)]
+
+
+@pytest.mark.parametrize("case", CASES, ids=[f"{c[0]}x{c[1]}:{c[2]}-D{c[3]}-{c[4]}blk-kv{c[5]}" for c in CASES])
+def test_both_routes_vs_oracle(dev, case):
+    B, hq, hkv, d, maxb, kv = case
+    rng = np.random.default_rng(B + maxb)
+    top = 16 * maxb
+    q, k, v, bt, sl = random_case(rng, B, hq, hkv, d, (1 if B > 1 else top - 3, top), max_blocks=maxb, neg_blocks=1)
+    if B > 2:
+        sl[0], sl[1] = top, 0
+        bt[0] = rng.permutation(k.shape[0])[:maxb]
+    qb = O.encode(q, O.BF16)
+    bf = torch.bfloat16
+    opts = {}
+    if kv == O.BF16:
+        kb, vb = O.encode(k, kv), O.encode(v, kv)
+        kc, vc = t16(kb, bf, dev), t16(vb, bf, dev)
+    else:
+        kb, vb = (O.encode((x / np.float32(0.02)).astype(np.float32), kv) for x in (k, v))
+        kc, vc = t8(kb, dev), t8(vb, dev)
+        opts = dict(kv_dtype=rllm_amd.DTYPE_FP8_E4M3 if kv == O.FP8_E4M3 else rllm_amd.DTYPE_FP8_E5M2,
+                    k_scale=0.02, v_scale=0.02)
+    scale = 1 / np.sqrt(d)
+    args = (t16(qb, bf, dev), kc, vc, ti(bt, torch.int32, dev), ti(sl, torch.int32, dev), scale)
+    log_case(f"decode routes {case}")
+    a = ops.paged_decode(*args, **opts)
+    again = ops.paged_decode(*args, **opts)
+    ws = torch.zeros(max(16, decode_workspace_size(B, hq, hkv, d, 16, maxb)), dtype=torch.uint8, device=dev)
+    b = ops.paged_decode(*args, workspace=ws, **opts)
+    torch.cuda.synchronize()
+    s = 0.02 if kv != O.BF16 else 1.0
+    ref = O.paged_attention_decode(qb, O.BF16, kb, vb, kv, bt, sl, scale, s, s, precision=1)
+    tol = TOL_BF16 if kv == O.BF16 else TOL_FP8
+    assert_close(f32(a), ref, tol, f"automatic {case}")
+    assert_close(f32(b), ref, tol, f"stream {case}")
+    assert torch.equal(a.view(torch.int16), again.view(torch.int16))
