@@ -1438,7 +1438,12 @@ int64_t stream_waves(int64_t num_seqs, int64_t hkv, int64_t max_blocks, int64_t 
     if (per_simd > 0)
         per_wave = std::min(per_wave,
                             std::max(STREAM_BLOCKS_PER_WAVE_MIN, (work_bound + per_simd - 1) / per_simd));
-    int64_t nw = (work_bound + per_wave - 1) / per_wave;
+    // whole waves per row: in a batch of equal lengths no wave then crosses from
+    // one row into the next, which costs it a second start and both rows a
+    // merge (32/8 heads, D 128, kernel us: 1 x 700 tokens 16.0 -> 12.3, 1 x 4000
+    // 32.0 -> 16.7, 8 x 1000 19.1 -> 13.8, 8 x 2500 30.1 -> 20.7; lengths spread
+    // over 1 : 32 within a few percent)
+    int64_t nw = num_seqs * hkv * ((max_blocks + per_wave - 1) / per_wave);
     const int64_t cap = one_per_simd && per_simd > 0 ? per_simd : resident;
     if (nw > cap) nw = cap;
     return nw < 1 ? 1 : nw;

@@ -125,29 +125,30 @@ GenArgs gen_args(void* out, const void* q, const void* kc, const void* vc, const
 }
 
 // Where the general decode beats the stream decode on the stream's own shapes
-// (block size 16, G = 1, 2, 4, 8): few rows, so that four waves a row and part
-// still leave CUs free, and
-//   - tables below 8 blocks, where a stream wave walks several rows in turn
-//     (a 4-block table is an even split and stays with it for G <= 2);
-//   - G = 8, whose stream waves carry 8 heads of vector work: up to 512 tokens,
-//     or long contexts;
-//   - G = 4: one 512-token part a row, or long contexts of few rows, which the
-//     stream cuts into at most one wave a 32 blocks.
-// Kernel us, stream / general, bf16, head_dim 128, sequences x tokens: G = 4
-// (32/8 heads) 8 x 32 19.8 / 8.7, 64 x 512 27.5 / 24.3, 1 x 16384 49.6 / 22.3, 4
-// x 8192 32.3 / 29.2; kept: 8 x 512 11.8 / 13.7, 64 x 1024 46.0 / 51.2, 8 x 4096
-// 28.4 / 29.0.  G = 8 (32/4) 8 x 64 18.7 / 9.1, 8 x 512 15.8 / 13.5, 1 x 32768
-// 99.8 / 25.2, 16 x 4096 32.6 / 29.1; E4M3, head_dim 64: kept 64 x 4096 41.7 /
-// 49.3.  G = 2 (16/8) 8 x 32 14.5 / 8.6; kept 8 x 256 9.4 / 11.5.  G = 1 (8/8) 8 x
-// 32 11.8 / 8.6; kept 8 x 64 8.0 / 9.2.
-bool general_decode_pays(int64_t units, int64_t g, int64_t maxb) {
+// (block size 16, G = 1, 2, 4, 8).  Both take a few round trips for a short
+// call; the stream's grow with lengths that differ (its equal shares then cut
+// rows unevenly) and with the heads a wave carries, the general kernel's with
+// the rows (four waves each).  Kernel us, stream / general, head_dim 128,
+// sequences x tokens (a : b: lengths drawn from a to b):
+//   G = 4 (32/8 heads), up to 512 tokens.  8 x 1:100 14.2 / 10.7, 8 x 9:300 14.5
+//     / 12.0, 40 x 14:450 15.9 / 15.9; equal lengths 8 x 100 9.8 / 10.9, 8 x 300
+//     11.6 / 12.0, 64 x 320 20.6 / 17.9.  Tables of 8, 16, 24 or 32 blocks
+//     split evenly and stay, unless the rows are many: 40 x 128 10.3 / 12.0, 8 x
+//     512 11.8 / 13.7, 64 x 512 27.5 / 24.3; so does one sequence below 8
+//     blocks: 1 x 32 7.8 / 8.7.
+//   G = 4, long contexts of few rows: 1 x 12000 37.4 / 20.8, 1 x 24000 52.4 /
+//     29.9, 3 x 7000 27.3 / 26.3, 3 x 125:4000 29.7 / 18.7; kept: 1 x 4000 16.7 /
+//     18.2, 5 x 4000 22.8 / 25.8, 8 x 7000 40.5 / 48.2.
+//   G = 8 (32/4): 8 x 64 18.7 / 9.1, 8 x 512 15.8 / 13.5, 1 x 32768 99.8 / 25.2, 16
+//     x 4096 32.6 / 29.1; E4M3, head_dim 64: kept 64 x 4096 41.7 / 49.3.
+bool general_decode_pays(int64_t seqs, int64_t hkv, int64_t g, int64_t maxb) {
+    const int64_t units = seqs * hkv, tokens = maxb * 16;
     if (units > 512) return false;
-    if (maxb < 8) return g >= 4 || maxb <= 2 || (g == 2 && maxb != 4);
-    const int64_t tokens = maxb * 16;
-    const bool few = units * tokens <= 262144;
-    if (g >= 8) return tokens <= 512 || (tokens >= 4096 && few);
-    if (g == 4) return (tokens > 256 && tokens <= 512 && units >= 256) || (tokens >= 8192 && few);
-    return false;
+    if (g >= 8) return maxb <= 32 || (tokens >= 4096 && units * tokens <= 262144);
+    if (g != 4) return false;
+    if (maxb <= 32) return maxb % 8 ? seqs > 1 || maxb > 8 : maxb >= 16 && units >= 500;
+    if (tokens >= 6144) return units * tokens <= 262144;
+    return tokens >= 3900 && units * tokens >= 40000 && units * tokens <= 131072;
 }
 
 }  // namespace
@@ -156,7 +157,7 @@ bool general_decode(void* out, const void* q, const void* kc, const void* vc, co
                     const int32_t* seq_lens, int64_t num_seqs, int64_t hq, int64_t hkv, int64_t d, int64_t maxb,
                     float scale, int32_t q_dtype, int32_t kv_dtype, float k_scale, float v_scale, hipStream_t stream,
                     int32_t* rc) {
-    if (!general_decode_pays(num_seqs * hkv, hq / hkv, maxb)) return false;
+    if (!general_decode_pays(num_seqs, hkv, hq / hkv, maxb)) return false;
     const bool fp8 = kv_dtype == KIND_FP8_E4M3 || kv_dtype == KIND_FP8_E5M2;
     GenArgs g = gen_args(out, q, kc, vc, bt, seq_lens, nullptr, num_seqs, num_seqs, hq, hkv, d, 16, maxb, scale, fp8,
                          k_scale, v_scale);
