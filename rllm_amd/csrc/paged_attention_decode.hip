@@ -1427,8 +1427,10 @@ int max_resident_waves() {
 // 70.2 us).  FP8 caches keep two: a wave spends twice the vector work per
 // byte on converting, which the second wave hides (config 3 196.6 against
 // 233.8 us at one per SIMD).
+// whole_rows: false gives the equal shares that ignore row ends, never more waves
+// than whole rows.
 int64_t stream_waves(int64_t num_seqs, int64_t hkv, int64_t max_blocks, int64_t resident,
-                     int64_t simds, bool one_per_simd) {
+                     int64_t simds, bool one_per_simd, bool whole_rows = true) {
     const int64_t work_bound = num_seqs * hkv * max_blocks;
     int64_t per_wave =
         std::min(STREAM_BLOCKS_PER_WAVE_MAX, std::max(STREAM_BLOCKS_PER_WAVE_MIN, max_blocks / 4));
@@ -1443,7 +1445,8 @@ int64_t stream_waves(int64_t num_seqs, int64_t hkv, int64_t max_blocks, int64_t 
     // merge (32/8 heads, D 128, kernel us: 1 x 700 tokens 16.0 -> 12.3, 1 x 4000
     // 32.0 -> 16.7, 8 x 1000 19.1 -> 13.8, 8 x 2500 30.1 -> 20.7; lengths spread
     // over 1 : 32 within a few percent)
-    int64_t nw = num_seqs * hkv * ((max_blocks + per_wave - 1) / per_wave);
+    int64_t nw = whole_rows ? num_seqs * hkv * ((max_blocks + per_wave - 1) / per_wave)
+                            : (work_bound + per_wave - 1) / per_wave;
     const int64_t cap = one_per_simd && per_simd > 0 ? per_simd : resident;
     if (nw > cap) nw = cap;
     return nw < 1 ? 1 : nw;
@@ -1581,13 +1584,6 @@ int32_t decode_impl(void* out, const void* q, const void* kc, const void* vc, co
     if (!specialised_shape(hq, hkv, d, bs))
         return generic_attention(out, q, kc, vc, bt, seq_lens, nullptr, num_seqs, num_seqs, hq, hkv, d, bs, maxb,
                                  scale, q_dtype, kv_dtype, k_scale, v_scale, !fixed_scratch, as_stream(stream));
-    // automatic plan without a caller's workspace: short tables and few rows
-    // may run the shape-general kernels
-    int32_t general_rc = 0;
-    if (partition_size == 0 && !workspace && !fixed_scratch &&
-        general_decode(out, q, kc, vc, bt, seq_lens, num_seqs, hq, hkv, d, maxb, scale, q_dtype, kv_dtype, k_scale,
-                       v_scale, as_stream(stream), &general_rc))
-        return general_rc;
     Kernels kern;
     RLLM_CHECK_ARG(pick_kernels(q_dtype, kv_dtype, d, G, &kern));
 
@@ -1599,10 +1595,30 @@ int32_t decode_impl(void* out, const void* q, const void* kc, const void* vc, co
         const int max_waves = max_resident_waves();
         if (max_waves < res) return (int32_t)hipErrorInvalidDevice;
         const bool fp8_kv = kv_dtype == KIND_FP8_E4M3 || kv_dtype == KIND_FP8_E5M2;
-        plan.num_waves =
-            static_cast<int32_t>(stream_waves(num_seqs, hkv, maxb, res, 4 * int64_t(device_cus()), !fp8_kv));
-        plan.max_waves = max_waves;
-        plan.ws_bytes = plan.num_waves > 1 ? stream_ws_bytes(max_waves, plan.num_waves, G, d) : 0;
+        auto waves = [&](bool whole_rows) {
+            plan.num_waves = static_cast<int32_t>(
+                stream_waves(num_seqs, hkv, maxb, res, 4 * int64_t(device_cus()), !fp8_kv, whole_rows));
+            plan.max_waves = max_waves;
+            plan.ws_bytes = plan.num_waves > 1 ? stream_ws_bytes(max_waves, plan.num_waves, G, d) : 0;
+        };
+        waves(true);
+        // a workspace sized for a larger call may fall short of whole rows (their
+        // count does not always grow with the batch): equal shares then
+        if (workspace && workspace_bytes < plan.ws_bytes) waves(false);
+        // without a caller's workspace short tables and few rows may run the
+        // shape-general kernels.  The stream's scratch is reserved all the
+        // same: a later capture of a smaller call may run the stream, and
+        // cannot allocate it
+        int32_t general_rc = 0;
+        if (!workspace && !fixed_scratch &&
+            general_decode(out, q, kc, vc, bt, seq_lens, num_seqs, hq, hkv, d, maxb, scale, q_dtype, kv_dtype,
+                           k_scale, v_scale, as_stream(stream), &general_rc)) {
+            void* reserved = nullptr;
+            if (!general_rc && plan.ws_bytes > 0 &&
+                g_workspaces.get(stream, WS_DECODE_STREAM, plan.ws_bytes, true, &reserved))
+                (void)hipGetLastError();
+            return general_rc;
+        }
     } else {
         RLLM_CHECK_ARG(make_partition_plan(num_seqs, hq, d, maxb, partition_size, &plan));
         RLLM_CHECK_ARG(num_seqs * hkv * plan.max_parts <= INT32_MAX);
@@ -1642,6 +1658,19 @@ int32_t decode_impl(void* out, const void* q, const void* kc, const void* vc, co
             const int role = plan.mode == Mode::Stream ? WS_DECODE_STREAM : WS_DECODE_PARTS;
             int32_t rc = g_workspaces.get(stream, role, plan.ws_bytes, plan.mode == Mode::Stream, &ws);
             if (rc) return rc;
+            if (!ws && plan.mode == Mode::Stream) {
+                // capturing: scratch of a larger call may still hold equal shares
+                const bool fp8_kv = kv_dtype == KIND_FP8_E4M3 || kv_dtype == KIND_FP8_E5M2;
+                const int64_t nw = stream_waves(num_seqs, hkv, maxb, resident_waves(kern.stream, 1),
+                                                4 * int64_t(device_cus()), !fp8_kv, false);
+                const int64_t bytes = stream_ws_bytes(plan.max_waves, nw, G, d);
+                rc = g_workspaces.get(stream, role, bytes, true, &ws);
+                if (rc) return rc;
+                if (ws) {
+                    plan.num_waves = static_cast<int32_t>(nw);
+                    plan.ws_bytes = bytes;
+                }
+            }
             if (!ws) {
                 // capturing on a stream whose scratch is missing or too small:
                 // one wave per (sequence, kv head), which needs none

@@ -56,3 +56,24 @@ def test_both_routes_vs_oracle(dev, case):
     assert_close(f32(a), ref, tol, f"automatic {case}")
     assert_close(f32(b), ref, tol, f"stream {case}")
     assert torch.equal(a.view(torch.int16), again.view(torch.int16))
+
+
+def test_workspace_of_a_larger_batch_serves_a_smaller(dev):
+    """Whole waves per row want more scratch for 15 rows of this width than for 16
+    (1035 waves against 1024): a workspace sized for the larger batch still runs
+    the smaller, on equal shares."""
+    hq, hkv, d, maxb = 4, 1, 64, 2048
+    have = decode_workspace_size(16, hq, hkv, d, 16, maxb)
+    assert have < decode_workspace_size(15, hq, hkv, d, 16, maxb)
+    rng = np.random.default_rng(15)
+    q, k, v, bt, sl = random_case(rng, 15, hq, hkv, d, (1, 700), max_blocks=maxb)
+    qb = O.encode(q, O.BF16)
+    kb, vb = (O.encode((x / np.float32(0.02)).astype(np.float32), O.FP8_E4M3) for x in (k, v))
+    ws = torch.zeros(have, dtype=torch.uint8, device=dev)
+    log_case("decode 15 rows, workspace of 16")
+    out = ops.paged_decode(t16(qb, torch.bfloat16, dev), t8(kb, dev), t8(vb, dev), ti(bt, torch.int32, dev),
+                           ti(sl, torch.int32, dev), 1 / 8, workspace=ws, kv_dtype=rllm_amd.DTYPE_FP8_E4M3,
+                           k_scale=0.02, v_scale=0.02)
+    torch.cuda.synchronize()
+    ref = O.paged_attention_decode(qb, O.BF16, kb, vb, O.FP8_E4M3, bt, sl, 1 / 8, 0.02, 0.02, precision=1)
+    assert_close(f32(out), ref, TOL_FP8, "workspace of a larger batch")

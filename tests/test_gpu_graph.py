@@ -311,3 +311,42 @@ def _replay_after_growth(small, big, st):
             call(big, out_big)   # eager work between replays, on the grown buffer
         torch.cuda.synchronize()
         assert_close(f32(out_big), big["ref"], TOL_BF16, f"eager call {r} after replay")
+
+
+def test_capture_after_a_larger_call_on_the_general_kernels(dev):
+    """One sequence of 24000 tokens runs the shape-general kernels, one of 4000
+    the stream.  After an eager call of the larger, a capture of the smaller
+    still finds the stream's scratch: its bits are those of an eager call, not of
+    the one-wave-per-row plan a capture without scratch falls back to."""
+    small = _decode_case(dev, 213, 1, (4000, 4000))
+    big = _decode_case(dev, 214, 1, (24000, 24000))
+    with RawStream() as st:
+        _capture_small_after_big(small, big, st)
+
+
+def _capture_small_after_big(small, big, st):
+    def call(x, out):
+        ops.paged_decode(x["q"], x["kc"], x["vc"], x["bt"], x["sl"], x["scale"], out=out, validate=False)
+
+    eager = torch.zeros_like(small["q"])
+    call(small, eager)           # on the current stream
+    out_big = torch.zeros_like(big["q"])
+    torch.cuda.synchronize()
+    log_case("graph decode: eager call of 24000 tokens")
+    with torch.cuda.stream(st):
+        call(big, out_big)
+    torch.cuda.synchronize()
+    assert_close(f32(out_big), big["ref"], TOL_BF16, "larger eager call vs oracle")
+    out = torch.zeros_like(small["q"])
+    g = torch.cuda.CUDAGraph()
+    log_case("graph decode: capture of 4000 tokens")
+    with torch.cuda.graph(g, stream=st):
+        call(small, out)
+    torch.cuda.synchronize()
+    for r in range(3):
+        out.zero_()
+        with torch.cuda.stream(st):
+            g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), eager.view(torch.int16)), f"replay {r}"
+    assert_close(f32(out), small["ref"], TOL_BF16, "replay vs oracle")
