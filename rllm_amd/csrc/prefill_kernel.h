@@ -236,6 +236,7 @@ template <int QT>
 __device__ __forceinline__ int longest_tile(int num_seqs, int lane, int n, int ctx, int rank, int& tile) {
     static_assert((QT & (QT - 1)) == 0, "tiles are counted by shifts");
     constexpr int SH = __builtin_ctz(QT);
+    ctx = min(ctx, 1 << 30);   // past any table: the same order, and the steps below stay in range
     // tiles of a sequence with more than thr keys: its last ones (tile i sees
     // ctx - n + min((i + 1) QT, n) keys)
     auto above = [](int n, int ctx, int thr) {

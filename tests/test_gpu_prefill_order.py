@@ -57,6 +57,26 @@ def test_prefill_order_vs_oracle(dev, case):
     assert_close(f32(out), ref, TOL_BF16, f"prefill order {case}")
 
 
+def test_context_past_the_table(dev):
+    """A context far past the table is clamped to it, however long it claims to
+    be: every query then sees the whole table, in the longest-first grid too."""
+    q, k, v, bt, sl, qsl = _case(9, 32, 32, 64, 300, 0, 5)
+    bf = torch.bfloat16
+    bt = np.where(bt < 0, 0, bt).astype(np.int32)
+    outs = []
+    for top in (1 << 24, 2**31 - 1):
+        sl[:] = top
+        log_case(f"prefill order, context {top} on a table of {bt.shape[1]} blocks")
+        outs.append(ops.paged_prefill(t16(q, bf, dev), t16(k, bf, dev), t16(v, bf, dev), ti(bt, torch.int32, dev),
+                                      ti(sl, torch.int32, dev), ti(qsl, torch.int32, dev), 1 / np.sqrt(64),
+                                      validate=False, out=torch.zeros_like(t16(q, bf, dev))))
+    torch.cuda.synchronize()
+    sl[:] = 1 << 24
+    ref = O.paged_attention_prefill(q, O.BF16, k, v, O.BF16, bt, sl, qsl, 1 / 8, precision=1)
+    assert_close(f32(outs[0]), ref, TOL_BF16, "context past the table")
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
 # prefix splits: the rule's 1, 2, 3 and the prefill rule's count
 @pytest.mark.parametrize("seqs,prefix,own", [(160, 16, 40), (128, 64, 16), (128, 128, 16), (32, 40, 3)])
 def test_prefix_splits_match_the_plain_decode(dev, seqs, prefix, own, monkeypatch):
