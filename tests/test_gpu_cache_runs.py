@@ -10,6 +10,7 @@ import oracle as O
 import rllm_amd
 from gpu_util import bits16, log_case, t16, t8, ti
 from rllm_amd import ops
+from test_gpu_rope_cache import _run as rope_run
 
 pytestmark = pytest.mark.gpu
 
@@ -84,3 +85,16 @@ def test_cache_write_unaligned_rows_take_the_token_kernel(dev):
     ek, ev = kc.copy(), kc.copy()
     O.cache_write(ek, ev, nk, nk, sl, bs, O.F16, O.F16)
     assert np.array_equal(bits16(gk), ek) and np.array_equal(bits16(gv), ev)
+
+
+# (kv heads, head_dim, block size, tokens): whole and part groups, one token past a
+# group, a block size without 16-slot groups, the widest head
+ROPE_SHAPES = [(8, 128, 16, 384), (2, 64, 32, 433), (1, 16, 16, 31), (1, 96, 16, 17), (2, 80, 24, 100), (1, 512, 16, 150)]
+
+
+@pytest.mark.parametrize("shape", ROPE_SHAPES, ids=[f"{s[0]}x{s[1]}-bs{s[2]}-n{s[3]}" for s in ROPE_SHAPES])
+@pytest.mark.parametrize("cache", [O.BF16, O.FP8_E4M3, O.FP8_E5M2])
+def test_rope_cache_runs_bit_exact(dev, shape, cache):
+    hkv, d, bs, n = shape
+    sl, nb = _slots(np.random.default_rng(n + d), n, bs)
+    rope_run(dev, n, 2 * hkv, hkv, d, nb, bs, O.BF16, cache, slots=sl, ks=0.5, vs=0.37, rne=cache == O.FP8_E5M2)
