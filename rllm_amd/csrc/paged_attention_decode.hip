@@ -1782,9 +1782,7 @@ int32_t decode_prefix_impl(void* out, const void* q, const void* kc, const void*
     Kernels kern;
     RLLM_CHECK_ARG(pick_kernels(q_dtype, kv_dtype, d, G, &kern));
 
-    const bool fp8_kv = kv_dtype == KIND_FP8_E4M3 || kv_dtype == KIND_FP8_E5M2;
-    const int64_t S = prefix_partial_splits(num_seqs, hq, hkv, d, prefix_blocks,
-                                            num_seqs * hkv * (maxb - prefix_blocks) * bs * d * (fp8_kv ? 2 : 4));
+    const int64_t S = prefix_partial_splits(num_seqs, hq, hkv, prefix_blocks);
     // the suffix partitions: whole 512-token chunks, as few per partition as
     // keep the widest suffix within CASCADE_MAX_SUFFIX_PARTS partitions
     const int64_t rest_chunks = (maxb - prefix_blocks + SC_BLOCKS - 1) / SC_BLOCKS;

@@ -265,27 +265,16 @@ int32_t sync_after(int32_t rc) {
 // cascade runs that mode inside its own kernel (cascade_kernel,
 // paged_attention_decode.hip); these helpers size it.
 
-// The partials run beside the suffix decode, so fewer, longer workgroups leave
-// it more CUs and the reduction fewer partials: the fewest splits whose
-// workgroups (about PREFIX_WG_NS and PREFIX_TILE_NS a 64-key tile) still end
-// within 85% of the time the suffix's bytes take (about SUFFIX_GBPS; its
-// length is the table's, an upper bound).  Where none does, the prefix is what
-// the call waits for: the prefill rule (a split keeps at least 4 tiles).  32/8
-// heads, D 128, us with 1 / 2 / 3 splits / the prefill rule's: 128 sequences
-// on 64 + 16 blocks 37.7 / 32.9 / 33.6 / 33.9 (4), 128 on 128 + 16 57.0 / 38.9
-// / 34.4 / 41.4 (8), 64 on 64 + 16 35.0 / 26.1 / 23.6 / 21.5 (4).
-constexpr int64_t PREFIX_WG_NS = 7500, PREFIX_TILE_NS = 1750, PREFIX_TILE_NS_64 = 1200, SUFFIX_GBPS = 5000;
-
-int64_t prefix_partial_splits(int64_t num_seqs, int64_t hq, int64_t hkv, int64_t d, int64_t prefix_blocks,
-                              int64_t suffix_bytes) {
-    const int64_t most = prefill_splits(prefix_base_wgs(num_seqs, hq, hkv), prefix_blocks);
-    const int64_t tiles = (prefix_blocks + PF_NBT - 1) / PF_NBT;
-    const int64_t suffix_ns = suffix_bytes / SUFFIX_GBPS;
-    for (int64_t sp = 1; sp < most; ++sp) {
-        const int64_t ns = PREFIX_WG_NS + (d == 64 ? PREFIX_TILE_NS_64 : PREFIX_TILE_NS) * ((tiles + sp - 1) / sp);
-        if (ns * 20 <= suffix_ns * 17) return sp;
-    }
-    return most;
+// The prefill rule (a split keeps at least 4 of the prefix's 64-token tiles):
+// the partials run beside the suffix decode, so fewer, longer workgroups
+// leave it more CUs; 2-tile splits measured no faster (20.1 -> 21.0 us on
+// config 4a) and cost the reduction a partial more per row.  Splits by the
+// suffix's time (2 for 128 sequences on 64 + 16 blocks instead of 4) were
+// faster (33.6 -> 32.7 us) but a little further from the 64-bit result (2.71e-3
+// -> 2.74e-3), and wanted more scratch for a batch of 96 than for one of 128, so
+// that a capture after the larger call lost the cascade.
+int64_t prefix_partial_splits(int64_t num_seqs, int64_t hq, int64_t hkv, int64_t prefix_blocks) {
+    return prefill_splits(prefix_base_wgs(num_seqs, hq, hkv), prefix_blocks);
 }
 
 bool prefix_partials_supported(int64_t hq, int64_t hkv, int64_t d, int64_t bs, int32_t q_dtype, int32_t kv_dtype,

@@ -20,7 +20,7 @@ import torch
 
 import oracle as O
 import rllm_amd
-from gpu_util import f32, log_case, t16, t8, ti
+from gpu_util import RawStream, f32, log_case, t16, t8, ti
 from helpers import TOL_BF16, TOL_FP8, assert_close
 from rllm_amd import ops, workloads
 
@@ -293,3 +293,39 @@ def test_prefix_auto_choice_follows_the_rule(dev, monkeypatch, B, P, own, cascad
     assert np.array_equal(never, plain)
     assert np.array_equal(auto, forced if cascade else plain)
     assert np.max(np.abs(forced - plain)) <= 2 ** -7 * max(1.0, float(np.abs(plain).max()))
+
+
+@pytest.mark.parametrize("B", [96, 112])
+def test_capture_after_a_larger_batch_keeps_the_cascade(dev, B):
+    """The scratch that an eager call of 128 sequences leaves on a stream holds
+    the cascade of a smaller batch: captured there, it replays the bits of its
+    eager call, not the plain decode's."""
+    rng = np.random.default_rng(4200)
+    q, k, v, bt, sl = prefix_case(rng, 128, 32, 8, 128, 64, (256, 256))
+    kc, vc = (t16(O.encode(x, O.BF16), torch.bfloat16, dev) for x in (k, v))
+    qd, btd, sld = t16(O.encode(q, O.BF16), torch.bfloat16, dev), ti(bt, torch.int32, dev), ti(sl, torch.int32, dev)
+
+    def call(n, out):
+        return ops.paged_decode_prefix(qd[:n], kc, vc, btd[:n], sld[:n], 1 / np.sqrt(128), 64, out=out, validate=False)
+
+    log_case(f"cascade of {B} captured after 128")
+    eager = call(B, torch.empty_like(qd[:B]))
+    plain = ops.paged_decode(qd[:B], kc, vc, btd[:B], sld[:B], 1 / np.sqrt(128), validate=False)
+    out = torch.zeros_like(eager)
+    torch.cuda.synchronize()
+    with RawStream() as st:
+        with torch.cuda.stream(st):
+            call(128, torch.empty_like(qd))
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=st):
+            call(B, out)
+        for r in range(3):
+            out.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(st):
+                g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, eager), f"replay {r}"
+            call(B, torch.empty_like(eager))   # eager work between the replays
+    assert not torch.equal(eager, plain)       # the two differ, so the test tells them apart

@@ -77,7 +77,7 @@ def test_context_past_the_table(dev):
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
 
 
-# prefix splits: the rule's 1, 2, 3 and the prefill rule's count
+# prefixes in 1, 4, 8 and 2 splits
 @pytest.mark.parametrize("seqs,prefix,own", [(160, 16, 40), (128, 64, 16), (128, 128, 16), (32, 40, 3)])
 def test_prefix_splits_match_the_plain_decode(dev, seqs, prefix, own, monkeypatch):
     rng = np.random.default_rng(seqs + prefix)
