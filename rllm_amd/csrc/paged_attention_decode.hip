@@ -1640,6 +1640,7 @@ int32_t decode_impl(void* out, const void* q, const void* kc, const void* vc, co
     a.v_scale = fp8 ? v_scale : 1.0f;
 
     void* ws = workspace;
+    WorkspaceHold hold;   // of the split-K partials, until the reduction is queued
     if (fixed_scratch && ws && plan.mode != Mode::Stream) {
         // the fixed array keeps the stream kernel's arrival counters at offset
         // 0, and every stream-mode call expects them at zero: split-K partials
@@ -1656,7 +1657,8 @@ int32_t decode_impl(void* out, const void* q, const void* kc, const void* vc, co
             // library-owned scratch; the stream kernel's arrival counters must
             // start at zero (every call leaves them at zero)
             const int role = plan.mode == Mode::Stream ? WS_DECODE_STREAM : WS_DECODE_PARTS;
-            int32_t rc = g_workspaces.get(stream, role, plan.ws_bytes, plan.mode == Mode::Stream, &ws);
+            int32_t rc = g_workspaces.get(stream, role, plan.ws_bytes, plan.mode == Mode::Stream, &ws,
+                                          plan.mode == Mode::Stream ? nullptr : &hold);
             if (rc) return rc;
             if (!ws && plan.mode == Mode::Stream) {
                 // capturing: scratch of a larger call may still hold equal shares
@@ -1794,7 +1796,8 @@ int32_t decode_prefix_impl(void* out, const void* q, const void* kc, const void*
     const int64_t rows = num_seqs * hq;
     RLLM_CHECK_ARG(rows <= (int64_t(1) << 40) / (max_parts * (d + 2)));
     void* ws = nullptr;
-    int32_t rc = g_workspaces.get(stream, WS_DECODE_PREFIX, rows * max_parts * (d + 2) * 4, false, &ws);
+    WorkspaceHold hold;   // until the reduction is queued
+    int32_t rc = g_workspaces.get(stream, WS_DECODE_PREFIX, rows * max_parts * (d + 2) * 4, false, &ws, &hold);
     if (rc) return rc;
     if (!ws)   // capturing on a stream whose scratch is missing or too small
         return decode_impl(out, q, kc, vc, bt, seq_lens, num_seqs, hq, hkv, d, bs, maxb, scale, q_dtype, kv_dtype,

@@ -63,13 +63,14 @@ int gen_cus() {
 }
 
 // Scratch of a split call; false and parts = 1 where there is none to be had (a
-// capture on a stream without it, no memory left).
-bool gen_take_scratch(GenArgs* g, hipStream_t stream) {
+// capture on a stream without it, no memory left).  `hold` keeps it until the
+// merge is queued.
+bool gen_take_scratch(GenArgs* g, hipStream_t stream, WorkspaceHold* hold) {
     if (g->parts <= 1) return true;
     const int64_t slots = static_cast<int64_t>(g->rows) * g->hq * g->parts;
     void* ws = nullptr;
     const int32_t rc = g_workspaces.get(reinterpret_cast<uintptr_t>(stream), WS_GENERIC, slots * (g->d + 2) * 4, false,
-                                        &ws);
+                                        &ws, hold);
     if (rc) (void)hipGetLastError();
     if (rc || !ws) {
         g->parts = 1;
@@ -163,7 +164,8 @@ bool general_decode(void* out, const void* q, const void* kc, const void* vc, co
                          k_scale, v_scale);
     if (!gen_mfma_shape(g, kv_dtype)) return false;
     gen_decode_plan(&g, fp8);
-    if (!gen_take_scratch(&g, stream)) return false;
+    WorkspaceHold hold;
+    if (!gen_take_scratch(&g, stream, &hold)) return false;
     *rc = launch_gen_decode(g, q_dtype, kv_dtype, g.parts, stream);
     return true;
 }
@@ -181,11 +183,12 @@ int32_t generic_attention(void* out, const void* q, const void* kc, const void* 
     const bool fp8 = kv_dtype == KIND_FP8_E4M3 || kv_dtype == KIND_FP8_E5M2;
     GenArgs g = gen_args(out, q, kc, vc, bt, seq_lens, qsl, num_seqs, rows, hq, hkv, d, bs, maxb, scale, fp8, k_scale,
                          v_scale);
+    WorkspaceHold hold;
     const int64_t units = num_seqs * hkv * ((hq / hkv + 15) / 16);
     if (!qsl && gen_mfma_shape(g, kv_dtype) && units <= INT32_MAX) {
         gen_decode_plan(&g, fp8);
         if (!may_allocate) g.parts = 1;
-        gen_take_scratch(&g, stream);
+        gen_take_scratch(&g, stream, &hold);
         return launch_gen_decode(g, q_dtype, kv_dtype, g.parts, stream);
     }
     if (qsl && gen_mfma_shape(g, kv_dtype) && hq / hkv <= 128) {
@@ -193,7 +196,7 @@ int32_t generic_attention(void* out, const void* q, const void* kc, const void* 
         if (base_wgs <= INT32_MAX / 8) {
             gen_prefill_plan(&g, base_wgs);
             if (!may_allocate) g.parts = 1;
-            gen_take_scratch(&g, stream);
+            gen_take_scratch(&g, stream, &hold);
             return launch_gen_prefill(g, q_dtype, kv_dtype, base_wgs, stream);
         }
     }

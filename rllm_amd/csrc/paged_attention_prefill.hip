@@ -201,12 +201,14 @@ int32_t prefill_impl(void* out, const void* q, const void* kc, const void* vc, c
     a.longest_first = splits == 1 && nwg > device_cu_count() && num_seqs <= LONGEST_MAX_SEQS;
     const int64_t rows = num_tokens * hq;
     int64_t splits_used = splits;
+    WorkspaceHold hold;   // until the merge is queued
     if (splits > 1) {
         RLLM_CHECK_ARG(nwg * splits <= INT32_MAX && rows <= (int64_t(1) << 40) / (splits * (d + 2)));
         void* ws = nullptr;
         // nullptr while capturing on a stream whose scratch is missing or too
         // small: the call then runs unsplit
-        const int32_t wrc = g_workspaces.get(stream, WS_PREFILL_SPLITS, rows * splits * (d + 2) * 4, false, &ws);
+        const int32_t wrc = g_workspaces.get(stream, WS_PREFILL_SPLITS, rows * splits * (d + 2) * 4, false, &ws,
+                                             &hold);
         if (wrc) return wrc;
         if (ws) {
             a.part_o = static_cast<float*>(ws);

@@ -1,4 +1,4 @@
-"""Calls from two host threads on two streams at once.
+"""Calls from two host threads at once, on two streams and on one.
 
 The library keeps its scratch per (device, stream): the stream decode's arrival
 counters and partials, the prefill's KV-split partials, the cascade's partials.
@@ -6,7 +6,10 @@ Two threads that call the decode, the chunked prefill, the mixed step and the
 cascade on their own streams at the same time must therefore give the bits
 that the same calls give one at a time, and the library's host state (scratch
 table, occupancy cache) must stand concurrent callers.  The ctypes calls
-release the GIL, so the two threads are inside the library together."""
+release the GIL, so the two threads are inside the library together.
+
+On one stream the threads share the scratch: a call of two launches (partials,
+then their merge) must not have the other thread's launches between its own."""
 import threading
 
 import numpy as np
@@ -127,3 +130,79 @@ def test_two_threads_on_two_streams_give_the_same_bits(dev, monkeypatch):
     for i in range(2):
         for j, name in enumerate(names):
             assert torch.equal(outs[i][j], ref[j]), f"{name} bits differ on thread {i}"
+
+
+def _two_launch_calls(rng, dev):
+    """One call of every path that leaves partials for a second launch: split-K
+    decode, shape-general decode (and a tuned shape that runs it), split prefill,
+    shape-general split prefill, cascade."""
+    c = _case(rng, dev)
+    bf = torch.bfloat16
+
+    def pool(n, hkv, d):
+        return [t16(O.encode(rng.standard_normal((n, hkv, d, 16)).astype(np.float32), O.BF16), bf, dev)
+                for _ in range(2)]
+
+    def q(n, hq, d):
+        return t16(O.encode(rng.standard_normal((n, hq, d)).astype(np.float32), O.BF16), bf, dev)
+
+    gk, gv = pool(200, 8, 96)
+    gq, gp = q(4, 24, 96), q(40, 24, 96)
+    gbt = ti(rng.integers(0, 200, (4, 190)).astype(np.int32), torch.int32, dev)
+    gsl = ti(np.array([3000, 1500, 2, 700], np.int32), torch.int32, dev)
+    psl = ti(np.array([1040], np.int32), torch.int32, dev)
+    pql = ti(np.array([0, 40], np.int32), torch.int32, dev)
+    lk, lv = pool(300, 2, 64)
+    lq = q(1, 8, 64)
+    lbt = ti(rng.integers(0, 300, (1, 500)).astype(np.int32), torch.int32, dev)
+    lsl = ti(np.array([7990], np.int32), torch.int32, dev)
+    kw = dict(validate=False)
+    return [
+        (c["dq"], lambda o, s: ops.paged_decode(c["dq"], c["kc"], c["vc"], c["dbt"], c["dsl"], c["scale"],
+                                                partition_size=512, out=o, stream=s, **kw)),
+        (gq, lambda o, s: ops.paged_decode(gq, gk, gv, gbt, gsl, 0.1, out=o, stream=s, **kw)),
+        (lq, lambda o, s: ops.paged_decode(lq, lk, lv, lbt, lsl, 0.125, out=o, stream=s, **kw)),
+        (c["pq"], lambda o, s: _prefill(c, o, s)),
+        (gp, lambda o, s: ops.paged_prefill(gp, gk, gv, gbt[:1], psl, pql, 0.1, out=o, stream=s, **kw)),
+        (c["cq"], lambda o, s: _cascade(c, o, s)),
+    ]
+
+
+def test_two_threads_on_one_stream_give_the_same_bits(dev, monkeypatch):
+    monkeypatch.setenv("RLLM_CASCADE", "always")
+    calls = [_two_launch_calls(np.random.default_rng(61 + i), dev) for i in range(2)]
+    refs = []
+    for mine in calls:
+        refs.append([torch.zeros_like(q) for q, _ in mine])
+        for (_, call), out in zip(mine, refs[-1]):
+            call(out, None)
+    outs = [[torch.zeros_like(r) for r in ref] for ref in refs]
+    wrong = [torch.zeros(len(ref), dtype=torch.int64, device=dev) for ref in refs]
+    torch.cuda.synchronize()
+    errors = []
+    start = threading.Barrier(2)
+
+    def worker(i, stream):
+        try:
+            start.wait()
+            with torch.cuda.stream(stream):
+                for _ in range(40):
+                    for (_, call), out in zip(calls[i], outs[i]):
+                        call(out, stream)
+                    for j, out in enumerate(outs[i]):
+                        wrong[i][j] += (out != refs[i][j]).any()
+                        out.zero_()
+        except Exception as e:   # reported by the main thread
+            errors.append(e)
+
+    with RawStream() as st:
+        threads = [threading.Thread(target=worker, args=(i, st)) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join(timeout=120)
+        assert not any(t.is_alive() for t in threads), "a worker thread did not finish"
+        torch.cuda.synchronize()
+    assert not errors, errors
+    for i in range(2):
+        assert wrong[i].tolist() == [0] * len(refs[i]), f"calls that differ, of 40, on thread {i}"
