@@ -292,12 +292,12 @@ __global__ __launch_bounds__(256, (gd_waves_per_simd<KVKIND, DP>())) void gen_de
                 a.part_ml[2 * slot + 1] = L;
             }
         } else {
-            const gm_f32x4 v = acc * (L > 0.f ? a.v_scale / L : 0.f);
+            const gm_f32x4 v = acc * gen_inv(a.v_scale, L);
             uint2 u;
             u.x = M::pack2(v[0], v[1]);
             u.y = M::pack2(v[2], v[3]);
             *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.out) + orow * D + d0) = u;
-            if (!(gen_finite(L) && gen_finite(v[0]) && gen_finite(v[1]) && gen_finite(v[2]) && gen_finite(v[3]))) {
+            if (!gen_stands(L, mx, gen_finite(v[0]) && gen_finite(v[1]) && gen_finite(v[2]) && gen_finite(v[3]))) {
                 bad_head[hd] = 1;
                 bad = true;
             }

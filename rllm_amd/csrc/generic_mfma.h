@@ -8,8 +8,10 @@
 // carries 16 (bf16) or 22 (f16) significant bits against the output's 8 / 11.
 // Two things the products do differently from a loop over the visible keys:
 // 0 * Inf (a masked key's value, or lo = 0) gives NaN, and so does Inf * -lo.
-// Both end in a non-finite output, so a row whose output or sum is not finite
-// is computed again by generic_row, whose answer stands.
+// Both end in a non-finite output, so a row whose output is not finite is
+// computed again by generic_row, whose answer stands.  Where the sum of the
+// weights is NaN (a visible score that is NaN or +inf) every output of the row
+// is, and is stored as such.
 #pragma once
 
 #include "generic_row.h"
@@ -116,6 +118,18 @@ __device__ __forceinline__ void gen_split8(const float (&p)[8], uint4& hi, uint4
 
 __device__ __forceinline__ bool gen_finite(float x) { return __builtin_fabsf(x) < INFINITY; }
 
+// factor of a row's outputs by the sum of its weights: 0 where it attended
+// nothing; NaN goes on
+__device__ __forceinline__ float gen_inv(float v_scale, float L) { return L == 0.f ? 0.f : v_scale / L; }
+
+// Whether a row's outputs stand, or generic_row computes the row again.  m is
+// the row's max as rounded, and a weight is taken relative to it from the exact
+// product: past 2^31 the rounding alone can put the largest weight at 0 or inf,
+// which leaves a sum of 0 under a max that was seen, or of inf.
+__device__ __forceinline__ bool gen_stands(float L, float m, bool finite) {
+    return L != L || (gen_finite(L) && finite && (L != 0.f || m == -INFINITY));
+}
+
 // Merges the parts of every row (row * hq + head): one wave per row, four rows
 // per workgroup.  Partials are unnormalised (sum of p v, relative to the
 // part's max); the parts are added in their order, so repeated calls give the
@@ -164,9 +178,8 @@ __global__ __launch_bounds__(256) void gen_merge_kernel(GenArgs a) {
                 if (p0 + i < np && fp != 0.f) acc += fp * v[i];
             }
         }
-        const float inv = L > 0.f ? a.v_scale / L : 0.f;
-        const gm_f32x4 o = acc * inv;
-        ok = gen_finite(L) && gen_finite(o[0]) && gen_finite(o[1]) && gen_finite(o[2]) && gen_finite(o[3]);
+        const gm_f32x4 o = acc * gen_inv(a.v_scale, L);
+        ok = gen_stands(L, mx, gen_finite(o[0]) && gen_finite(o[1]) && gen_finite(o[2]) && gen_finite(o[3]));
         if (d0 < D) {
             uint2 u;
             u.x = M::pack2(o[0], o[1]);

@@ -305,11 +305,10 @@ __global__ __launch_bounds__(256, DP <= 128 ? 2 : 1) void gen_prefill_kernel(Gen
             }
         return;
     }
-    const float inv = l > 0.f ? a.v_scale / l : 0.f;
+    const float inv = gen_inv(a.v_scale, l);
     bool ok = true;
     if (live) {
         uint16_t* dst = static_cast<uint16_t*>(a.out) + orow * D;
-        ok = gen_finite(l);
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
@@ -327,6 +326,7 @@ __global__ __launch_bounds__(256, DP <= 128 ? 2 : 1) void gen_prefill_kernel(Gen
                 w.y = M::pack2(x[2], x[3]);
                 *reinterpret_cast<uint2*>(dst + d0) = w;
             }
+        ok = gen_stands(l, m_run, ok);
     }
     const uint64_t bad = __builtin_amdgcn_ballot_w64(!ok);
     if (hl == 0) bad_row[m] = static_cast<int>(((bad >> l32) | (bad >> (l32 + 32))) & 1);

@@ -53,6 +53,13 @@ __device__ __forceinline__ float kv_elem(const void* base, int64_t i) {
     }
 }
 
+// the rounded product: fused into the subtraction of the max, which was rounded,
+// it would leave a score past 2^31 a weight of 0 or inf instead of 1
+__device__ __forceinline__ float rounded_mul(float a, float b) {
+#pragma clang fp contract(off)
+    return a * b;
+}
+
 // Attends row `row`, head `qh` with the whole workgroup and stores the output.
 // head_dim <= 64 * NJ (NJ dims a lane); `lds`: 8 + 4 * head_dim floats that no
 // thread of the workgroup still reads.
@@ -106,10 +113,12 @@ __device__ __forceinline__ void generic_row(const GenArgs& a, int64_t row, int q
                 const int d = lane + 64 * j;
                 if (d < D) dot += qv[j] * kv_elem<KVKIND>(a.kc, base + static_cast<int64_t>(d) * a.bs + off);
             }
-            const float sc = wave_sum(dot) * a.s_scale;   // log2 domain
+            const float sc = rounded_mul(wave_sum(dot), a.s_scale);   // log2 domain
             const float m_new = fmaxf(m, sc);
-            const float alpha = exp2f(m - m_new);
-            const float p = exp2f(sc - m_new);
+            // a score of -inf weighs nothing, whatever came before; NaN goes on
+            const float ms = m_new == -INFINITY ? 0.f : m_new;
+            const float alpha = exp2f(m - ms);
+            const float p = exp2f(sc - ms);
             l = l * alpha + p;
 #pragma unroll
             for (int j = 0; j < NJ; ++j) {
@@ -143,7 +152,8 @@ __device__ __forceinline__ void generic_row(const GenArgs& a, int64_t row, int q
         float acc = 0.f;
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc += f[i] * so[i * D + d];
-        orow[d] = from_f32<qtag>(L > 0.f ? acc / L * a.v_scale : 0.f);
+        // no weight at all: zeros; a NaN sum (a score that is NaN or +inf) goes on
+        orow[d] = from_f32<qtag>(L == 0.f ? 0.f : acc / L * a.v_scale);
     }
 }
 

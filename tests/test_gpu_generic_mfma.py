@@ -160,3 +160,67 @@ def test_prefill_value_that_is_not_finite_stays_in_its_rows(dev, bad, cached):
     assert ok[:37].all() and not ok[37:, 3:, 3].any()
     assert np.array_equal(np.isfinite(got), ok) and np.array_equal(np.isposinf(got), np.isposinf(ref))
     assert (np.abs(got[ok] - ref[ok]) <= 2e-2 + 1e-2 * np.abs(ref[ok])).all()
+
+
+# scores that are not finite: (head_dim, q heads, kv heads, block size, contexts)
+# on the scalar routine, the matrix cores in one part and in several, and the
+# stream decode's own shapes on both sides of the route
+SCORES = [(36, 3, 1, 16, [40, 90]), (96, 6, 2, 16, [40, 90]), (96, 6, 2, 16, [700, 1300]),
+          (128, 16, 2, 16, [40, 300]), (64, 4, 1, 16, [90, 6400]), (128, 4, 2, 16, [40, 90])]
+BAD = {"k nan": np.nan, "k +inf": np.inf, "k -inf": -np.inf, "q nan": np.nan, "q inf": np.inf, "overflow": 3e19}
+
+
+def _plant(bad, q_row, k_elem, fill):
+    """One q or K entry that is not finite, or a product past fp32's range."""
+    if bad[0] == "k":
+        k_elem[...] = fill
+    else:
+        q_row[5] = fill
+        if bad == "overflow":
+            q_row[6:] = 0
+            k_elem[...] = fill
+
+
+def _same_but_nan(got, ref, what):
+    assert np.array_equal(np.isnan(got), np.isnan(ref)), what
+    ok = ~np.isnan(ref)
+    assert np.isfinite(got[ok]).all() and (np.abs(got[ok] - ref[ok]) <= 2e-2 + 1e-2 * np.abs(ref[ok])).all(), what
+
+
+# (the stream decode's last shape without "q nan": a row that has no score but NaN
+# finds no max there and ends in zeros)
+DECODE_SCORES = [(c, b) for c in SCORES for b in BAD if c != SCORES[-1] or b != "q nan"]
+
+
+@pytest.mark.parametrize("case,bad", DECODE_SCORES,
+                         ids=[f"D{c[0]}-{c[1]}x{c[2]}-{c[4][1]}-{b.replace(' ', '-')}" for c, b in DECODE_SCORES])
+def test_decode_scores_that_are_not_finite(dev, case, bad):
+    # a visible score of NaN or +inf makes its row NaN, one of -inf weighs nothing
+    D, hq, hkv, bs, lens = case
+    rng = np.random.default_rng(17)
+    q, k, v, bt, sl = random_case(rng, 2, hq, hkv, D, (max(lens), max(lens)))
+    sl[:] = lens
+    _plant(bad, q[1, 0], k[bt[1, 2], 0, 5, 3:4], BAD[bad])
+    log_case(f"decode scores {case} {bad}")
+    got, _ = _decode(dev, (D, hq, hkv, bs, O.BF16, None), q, k, v, bt, sl, 1 / np.sqrt(D))
+    qb, kb, vb = (O.encode(x, O.BF16) for x in (q, k, v))
+    ref = O.paged_attention_decode(qb, O.BF16, kb, vb, O.BF16, bt, sl, 1 / np.sqrt(D), precision=0)
+    assert np.isnan(ref).any() or bad == "k -inf"
+    _same_but_nan(got, ref, f"{case} {bad}")
+
+
+@pytest.mark.parametrize("D,hq,hkv,cached", [(36, 3, 1, 20), (128, 6, 2, 0), (128, 6, 2, 700)])
+@pytest.mark.parametrize("bad", BAD, ids=[b.replace(" ", "-") for b in BAD])
+def test_prefill_scores_that_are_not_finite(dev, D, hq, hkv, cached, bad):
+    case = (D, hq, hkv, 16, O.BF16, [50], [cached])
+    rng = np.random.default_rng(18)
+    q, k, v, bt, sl, qsl = _prefill_case(rng, case)
+    bt[bt < 0] = np.setdiff1d(np.arange(k.shape[0]), bt)[0]
+    pos = cached + 17
+    _plant(bad, q[30, 0], k[bt[0, pos // 16], 0, 5, pos % 16:pos % 16 + 1], BAD[bad])
+    log_case(f"prefill scores {case} {bad}")
+    got, _ = _prefill(dev, O.BF16, q, k, v, bt, sl, qsl, 1 / np.sqrt(D))
+    qb, kb, vb = (O.encode(x, O.BF16) for x in (q, k, v))
+    ref = O.paged_attention_prefill(qb, O.BF16, kb, vb, O.BF16, bt, sl, qsl, 1 / np.sqrt(D), precision=0)
+    assert np.isnan(ref).any() and not np.isnan(ref[:17]).any() or bad == "k -inf"
+    _same_but_nan(got, ref, f"{case} {bad}")
