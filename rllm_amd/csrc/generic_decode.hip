@@ -208,8 +208,9 @@ __global__ __launch_bounds__(256, (gd_waves_per_simd<KVKIND, DP>())) void gen_de
                 if (!whole && !(vo[i] >= 0 && w0 + 8 * (4 * i + q4) + t < t_hi)) p[i][t] = -INFINITY;
                 mx = fmaxf(mx, p[i][t]);
             }
-        // c = 0 times an infinity must not poison the max
-        const float m_new = fmaxf(m_run, quad_max(mx == -INFINITY ? mx : mx * c));
+        // the max, lowered by the weights' lift; c = 0 times an infinity must not
+        // poison it
+        const float m_new = fmaxf(m_run, quad_max(mx == -INFINITY ? mx : fmaf(mx, c, -gen_decode_lift<QKIND>())));
         const float ms = m_new == -INFINITY ? 0.f : m_new;
         const float alpha = exp2f(m_run - ms);
         float sum = 0.f;

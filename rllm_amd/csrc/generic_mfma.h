@@ -2,10 +2,15 @@
 // (generic_decode.hip, generic_prefill.hip): element conversion, MFMA
 // wrappers, the two-term weights and the merge of split contexts.
 //
-// Both kernels keep the attention weights at the precision of the scalar row
-// routine: a weight p (fp32) enters the V product as the sum of two 16-bit
-// values, hi = round(p) and lo = round(p - hi), one product each.  The pair
-// carries 16 (bf16) or 22 (f16) significant bits against the output's 8 / 11.
+// A weight p (fp32) enters the V product as the sum of two 16-bit values, hi =
+// round(p) and lo = round(p - hi), one product each.  The pair carries 16 (bf16)
+// or 22 (f16) significant bits against the output's 8 / 11.  f16 has no range
+// below 2^-24: its weights are taken relative to 2^-lift times the row's max (the
+// sums carry the factor too, so it cancels), which puts the pair's last bit at
+// 2^-24 - lift of the largest weight.  Prefill lifts by 10, its fast softmax
+// letting weights grow to 48 before the max is taken again; decode by 15: with
+// values up to 65504 a weight's rounding then stays below f16's last bit.
+// Unlifted, a tail of weights at 2^-22 lost 11%, one below 2^-25 everything.
 // Two things the products do differently from a loop over the visible keys:
 // 0 * Inf (a masked key's value, or lo = 0) gives NaN, and so does Inf * -lo.
 // Both end in a non-finite output, so a row whose output is not finite is
@@ -88,6 +93,10 @@ __device__ __forceinline__ uint4 gen_to16(const GenRaw<KVKIND>& r) {
         return make_uint4(d[0], d[1], d[2], d[3]);
     }
 }
+
+// log2 of the factor of the weights (above)
+template <int QKIND> constexpr float gen_decode_lift() { return QKIND == KIND_F16 ? 15.f : 0.f; }
+template <int QKIND> constexpr float gen_prefill_lift() { return QKIND == KIND_F16 ? 10.f : 0.f; }
 
 // the first n of 8 16-bit values, the rest zeroed
 __device__ __forceinline__ uint4 gen_keep(uint4 w, int n) {

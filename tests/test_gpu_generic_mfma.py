@@ -224,3 +224,38 @@ def test_prefill_scores_that_are_not_finite(dev, D, hq, hkv, cached, bad):
     ref = O.paged_attention_prefill(qb, O.BF16, kb, vb, O.BF16, bt, sl, qsl, 1 / np.sqrt(D), precision=0)
     assert np.isnan(ref).any() and not np.isnan(ref[:17]).any() or bad == "k -inf"
     _same_but_nan(got, ref, f"{case} {bad}")
+
+
+@pytest.mark.parametrize("log2w", [-16.4, -20.4, -22.4, -25.4])
+@pytest.mark.parametrize("path", ["decode", "decode split", "prefill", "prefill split"])
+def test_f16_tail_of_small_weights(dev, path, log2w):
+    """One key outweighs a long flat tail 2^-log2w to 1 and is zero in half of the
+    head_dims, which then hold the tail's share alone: about n * 2^log2w of its
+    values.  Those outputs are f16 (2^-11 of their size); each weight is off by
+    half of its pair's last bit at most (2^-25 - lift of the largest weight), and by
+    what three fp32 roundings of the scale do to an exponent of 25 (under 2^-18) and
+    the exponential and the sums (2^-20)."""
+    D, hq, hkv = 96, 6, 2
+    split, pre = "split" in path, "prefill" in path
+    n = 2000 if split else 400
+    rng = np.random.default_rng(31)
+    q, k, v, bt, sl = random_case(rng, 1, hq, hkv, D, (n, n))
+    # scores: 8 * 8 * scale' for the key at position 3, none for the others
+    q[:], k[:] = 0, 0
+    q[..., 0] = 8
+    k[bt[0, 0], :, 0, 3] = 8
+    scale = -log2w * np.log(2) / 64
+    v[:] = np.abs(v) * 1024 + 512
+    v[bt[0, 0], :, :D // 2, 3] = 0
+    args = (bt, sl, scale)
+    log_case(f"f16 tail {path} 2^{log2w}")
+    if pre:
+        qsl = np.array([0, 3], np.int32)
+        got, ref = _prefill(dev, O.F16, np.repeat(q, 3, 0), k, v, bt, sl, qsl, scale)
+    else:
+        got, ref = _decode(dev, (D, hq, hkv, 16, O.F16, None), q, k, v, *args)
+    lift = 10 if pre else 15
+    rel = 2.0 ** -11 + 2.0 ** (-25 - lift - log2w) + 2.0 ** -17
+    got, ref = got[..., :D // 2], ref[..., :D // 2]
+    # f16's own subnormal step below 2^-14
+    assert (np.abs(got - ref) <= rel * np.abs(ref) + 2.0 ** -25).all(), np.abs(got / ref - 1).max()
