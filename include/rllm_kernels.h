@@ -28,10 +28,14 @@
  * size up to 4096 and num_q_heads a multiple of num_kv_heads.  head_dim 64 /
  * 128 with block_size 16 and num_q_heads / num_kv_heads in {1, 2, 4, 8} run
  * the tuned kernels; every other shape runs the shape-general kernels
- * (partition_size and the workspace argument are ignored; decode splits long
- * contexts over library-owned scratch per (device, stream) and runs unsplit
- * where there is none: during a capture on a stream that has no scratch yet,
- * through rllm_paged_attention_decode_noalloc, or when no memory is left).
+ * (partition_size is ignored).  They split long contexts over scratch, which
+ * is library-owned per (device, stream), and run unsplit where there is none: a
+ * decode captured on a stream that has no scratch yet, any captured prefill,
+ * rllm_paged_attention_decode_noalloc, or no memory left.  A decode that is
+ * given a workspace takes no library scratch: it splits over the workspace, past
+ * the arrival counters at its start, or, where that is too small, not at all
+ * (32 KiB + num_seqs * num_q_heads * 64 * (head_dim + 2) * 4 bytes always do;
+ * any non-null one, however small, keeps the library's scratch out).
  * Cache writes accept any shape.
  *
  * Differences from the reference kernels, all deliberate:

@@ -1579,11 +1579,20 @@ int32_t decode_impl(void* out, const void* q, const void* kc, const void* vc, co
     RLLM_CHECK_ARG(q_dtype == KIND_F16 || q_dtype == KIND_BF16);
     RLLM_CHECK_ARG(kv_dtype == q_dtype || kv_dtype == KIND_FP8_E4M3 || kv_dtype == KIND_FP8_E5M2);
     RLLM_CHECK_ARG(std::isfinite(scale) && std::isfinite(k_scale) && std::isfinite(v_scale));
-    // other head_dims, block sizes and GQA ratios: the shape-general kernel
-    // (no workspace; partition_size does not apply)
-    if (!specialised_shape(hq, hkv, d, bs))
+    // other head_dims, block sizes and GQA ratios: the shape-general kernels
+    // (partition_size does not apply).  A caller's workspace is used past the
+    // stream kernel's arrival counters, which calls of other shapes may keep there.
+    if (!specialised_shape(hq, hkv, d, bs)) {
+        char* gws = nullptr;
+        if (workspace && !fixed_scratch) {
+            const int64_t skip = stream_counter_bytes(max_resident_waves());
+            gws = static_cast<char*>(workspace) + skip;
+            workspace_bytes -= skip;
+        }
         return generic_attention(out, q, kc, vc, bt, seq_lens, nullptr, num_seqs, num_seqs, hq, hkv, d, bs, maxb,
-                                 scale, q_dtype, kv_dtype, k_scale, v_scale, !fixed_scratch, as_stream(stream));
+                                 scale, q_dtype, kv_dtype, k_scale, v_scale, !fixed_scratch, gws, workspace_bytes,
+                                 as_stream(stream));
+    }
     Kernels kern;
     RLLM_CHECK_ARG(pick_kernels(q_dtype, kv_dtype, d, G, &kern));
 
@@ -2095,7 +2104,7 @@ int64_t rllm_paged_attention_decode_workspace_size(int64_t num_seqs, int64_t num
         max_num_blocks_per_seq < 0 || head_dim < 1 || block_size < 1)
         return -1;
     if (!specialised_shape(num_q_heads, num_kv_heads, head_dim, block_size))
-        return head_dim <= 1024 ? 0 : -1;   // the shape-general kernel needs no workspace
+        return head_dim <= 1024 ? 0 : -1;   // the shape-general kernels need none (and use what they are given)
     if (partition_size == 0) {
         const int res = max_resident_waves();
         if (res <= 0) return -1;

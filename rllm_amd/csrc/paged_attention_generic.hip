@@ -62,23 +62,30 @@ int gen_cus() {
     return cus;
 }
 
-// Scratch of a split call; false and parts = 1 where there is none to be had (a
-// capture on a stream without it, no memory left).  `hold` keeps it until the
-// merge is queued.
-bool gen_take_scratch(GenArgs* g, hipStream_t stream, WorkspaceHold* hold) {
-    if (g->parts <= 1) return true;
-    const int64_t slots = static_cast<int64_t>(g->rows) * g->hq * g->parts;
-    void* ws = nullptr;
-    const int32_t rc = g_workspaces.get(reinterpret_cast<uintptr_t>(stream), WS_GENERIC, slots * (g->d + 2) * 4, false,
-                                        &ws, hold);
-    if (rc) (void)hipGetLastError();
-    if (rc || !ws) {
+bool gen_set_scratch(GenArgs* g, void* ws) {
+    if (!ws) {
         g->parts = 1;
         return false;
     }
     g->part_o = static_cast<float*>(ws);
-    g->part_ml = g->part_o + slots * g->d;
+    g->part_ml = g->part_o + static_cast<int64_t>(g->rows) * g->hq * g->parts * g->d;
     return true;
+}
+
+int64_t gen_scratch_bytes(const GenArgs& g) {
+    return static_cast<int64_t>(g.rows) * g.hq * g.parts * (g.d + 2) * 4;
+}
+
+// Library scratch of a split call; false and parts = 1 where there is none to be
+// had (a capture on a stream without it, no memory left).  `hold` keeps it until
+// the merge is queued.
+bool gen_take_scratch(GenArgs* g, hipStream_t stream, WorkspaceHold* hold) {
+    if (g->parts <= 1) return true;
+    void* ws = nullptr;
+    const int32_t rc = g_workspaces.get(reinterpret_cast<uintptr_t>(stream), WS_GENERIC, gen_scratch_bytes(*g), false,
+                                        &ws, hold);
+    if (rc) (void)hipGetLastError();
+    return gen_set_scratch(g, rc ? nullptr : ws);
 }
 
 // Decode: parts of whole 512-token rounds (one window for each of a
@@ -174,7 +181,7 @@ int32_t generic_attention(void* out, const void* q, const void* kc, const void* 
                           const int32_t* seq_lens, const int32_t* qsl, int64_t num_seqs, int64_t rows,
                           int64_t hq, int64_t hkv, int64_t d, int64_t bs, int64_t maxb, float scale,
                           int32_t q_dtype, int32_t kv_dtype, float k_scale, float v_scale, bool may_allocate,
-                          hipStream_t stream) {
+                          void* workspace, int64_t workspace_bytes, hipStream_t stream) {
     RLLM_CHECK_ARG(d >= 1 && d <= GEN_MAX_D && bs >= 1 && bs <= 4096);
     RLLM_CHECK_ARG(hq % hkv == 0 && hq <= 4096 && num_seqs <= (int64_t(1) << 30));
     RLLM_CHECK_ARG(maxb >= 0 && maxb * bs <= (int64_t(1) << 31) - 1);
@@ -187,15 +194,27 @@ int32_t generic_attention(void* out, const void* q, const void* kc, const void* 
     const int64_t units = num_seqs * hkv * ((hq / hkv + 15) / 16);
     if (!qsl && gen_mfma_shape(g, kv_dtype) && units <= INT32_MAX) {
         gen_decode_plan(&g, fp8);
-        if (!may_allocate) g.parts = 1;
-        gen_take_scratch(&g, stream, &hold);
+        if (workspace) {
+            const bool fits = gen_scratch_bytes(g) <= workspace_bytes && reinterpret_cast<uintptr_t>(workspace) % 16 == 0;
+            gen_set_scratch(&g, fits ? workspace : nullptr);
+        } else if (!may_allocate) {
+            g.parts = 1;
+        } else {
+            gen_take_scratch(&g, stream, &hold);
+        }
         return launch_gen_decode(g, q_dtype, kv_dtype, g.parts, stream);
     }
     if (qsl && gen_mfma_shape(g, kv_dtype) && hq / hkv <= 128) {
         const int64_t base_wgs = gen_prefill_base_wgs(g);
         if (base_wgs <= INT32_MAX / 8) {
             gen_prefill_plan(&g, base_wgs);
-            if (!may_allocate) g.parts = 1;
+            // Prefill has no workspace argument: a captured call is not split, so
+            // that graphs of one stream share no buffer and may be replayed on
+            // several.
+            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+            if (g.parts > 1 && (!may_allocate || hipStreamIsCapturing(stream, &cap) != hipSuccess ||
+                                cap != hipStreamCaptureStatusNone))
+                g.parts = 1;
             gen_take_scratch(&g, stream, &hold);
             return launch_gen_prefill(g, q_dtype, kv_dtype, base_wgs, stream);
         }

@@ -177,13 +177,13 @@ int32_t prefill_impl(void* out, const void* q, const void* kc, const void* vc, c
     // other head_dims, block sizes and GQA ratios: the shape-general kernel
     if (!specialised_shape(hq, hkv, d, bs))
         return generic_attention(out, q, kc, vc, bt, seq_lens, qsl, num_seqs, num_tokens, hq, hkv, d, bs, maxb,
-                                 scale, q_dtype, kv_dtype, k_scale, v_scale, true, as_stream(stream));
+                                 scale, q_dtype, kv_dtype, k_scale, v_scale, true, nullptr, 0, as_stream(stream));
 
     // f16 queries whose pre-scale could overflow: the shape-general kernel,
     // which scales the fp32 scores
     if (!q_prescale_ok(q_dtype, kv_dtype, scale, k_scale))
         return generic_attention(out, q, kc, vc, bt, seq_lens, qsl, num_seqs, num_tokens, hq, hkv, d, bs, maxb,
-                                 scale, q_dtype, kv_dtype, k_scale, v_scale, true, as_stream(stream));
+                                 scale, q_dtype, kv_dtype, k_scale, v_scale, true, nullptr, 0, as_stream(stream));
 
     const int64_t nwg = chunk_base_wgs(num_tokens, num_seqs, hq, hkv);
     RLLM_CHECK_ARG(nwg <= INT32_MAX);

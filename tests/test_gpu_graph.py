@@ -350,3 +350,105 @@ def _capture_small_after_big(small, big, st):
         torch.cuda.synchronize()
         assert torch.equal(out.view(torch.int16), eager.view(torch.int16)), f"replay {r}"
     assert_close(f32(out), small["ref"], TOL_BF16, "replay vs oracle")
+
+
+def _general_decode(dev, seed):
+    """24/8 heads of head_dim 96: a shape of the shape-general kernels, split."""
+    rng = np.random.default_rng(seed)
+    q, k, v, bt, sl = random_case(rng, 4, 24, 8, 96, (100, 3000))
+    sl[0] = 3000 - 16 * seed % 48
+    bf = torch.bfloat16
+    bt = rng.integers(0, k.shape[0], (4, 188)).astype(np.int32)
+    return dict(q=t16(O.encode(q, O.BF16), bf, dev), kc=t16(O.encode(k, O.BF16), bf, dev),
+                vc=t16(O.encode(v, O.BF16), bf, dev), bt=ti(bt, torch.int32, dev), sl=ti(sl, torch.int32, dev))
+
+
+def _replay_on_two_streams(graphs, outs, refs, what):
+    """Both graphs at once, each on its own stream, 20 times."""
+    with RawStream() as s0, RawStream() as s1:
+        for r in range(20):
+            for o in outs:
+                o.zero_()
+            torch.cuda.synchronize()
+            for g, s in zip(graphs, (s0, s1)):
+                with torch.cuda.stream(s):
+                    g.replay()
+            torch.cuda.synchronize()
+            for o, ref in zip(outs, refs):
+                assert torch.equal(o, ref), f"{what}: replay {r}"
+
+
+COUNTERS = 32 * 1024   # arrival counters at the start of a workspace
+
+
+def test_general_decode_takes_the_callers_workspace(dev):
+    """Shape-general decodes split over a caller's workspace, past the arrival
+    counters, and then share nothing: graphs captured on one stream give the
+    eager bits on two at once.  A workspace that is too small leaves the call
+    unsplit, as the entry point without scratch runs it."""
+    xs = [_general_decode(dev, seed) for seed in (5, 6)]
+
+    def call(x, out, **kw):
+        return ops.paged_decode(x["q"], x["kc"], x["vc"], x["bt"], x["sl"], 0.1, out=out, validate=False, **kw)
+
+    log_case("general decode, caller workspaces")
+    eager = [call(x, torch.empty_like(x["q"])) for x in xs]
+    size = COUNTERS + 4 * 24 * 64 * 98 * 4
+    spaces = [torch.zeros(size, dtype=torch.uint8, device=dev) for _ in xs]
+    outs = [torch.zeros_like(x["q"]) for x in xs]
+    small = call(xs[0], torch.empty_like(outs[0]), workspace=torch.zeros(16, dtype=torch.uint8, device=dev))
+    torch.cuda.synchronize()
+    assert not torch.equal(small, eager[0])       # other sums: not split
+    assert_close(f32(small), f32(eager[0]), TOL_BF16, "unsplit")
+    graphs = []
+    with RawStream() as st:
+        with torch.cuda.stream(st):
+            call(xs[0], torch.empty_like(outs[0]))   # the stream has library scratch, too
+        torch.cuda.synchronize()
+        for x, o, ws in zip(xs, outs, spaces):
+            graphs.append(torch.cuda.CUDAGraph())
+            with torch.cuda.graph(graphs[-1], stream=st):
+                call(x, o, workspace=ws)
+        torch.cuda.synchronize()
+        _replay_on_two_streams(graphs, outs, eager, "general decode")
+    for ws in spaces:
+        assert not ws[:COUNTERS].any() and ws[COUNTERS:].any()
+
+
+def test_general_prefill_graphs_share_nothing(dev):
+    """A captured shape-general prefill is not split, whatever scratch its stream
+    has: graphs of one stream give one another's bits on two at once."""
+    xs = [_general_decode(dev, seed) for seed in (7, 8)]
+    qsl = ti(np.array([0, 30], np.int32), torch.int32, dev)
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(3)
+    qs = [torch.randn((30, 24, 96), generator=gen, device=dev, dtype=torch.bfloat16) for _ in xs]
+
+    def call(i, out):
+        x = xs[i]
+        return ops.paged_prefill(qs[i], x["kc"], x["vc"], x["bt"][:1], x["sl"][:1], qsl, 0.1, out=out, validate=False)
+
+    log_case("general prefill, captured")
+    eager = [call(i, torch.empty_like(q)) for i, q in enumerate(qs)]
+    refs = []
+    for i, q in enumerate(qs):                     # captured where there is no scratch at all
+        out, g = torch.zeros_like(q), torch.cuda.CUDAGraph()
+        with RawStream() as fresh:
+            with torch.cuda.graph(g, stream=fresh):
+                call(i, out)
+            g.replay()
+            torch.cuda.synchronize()
+        refs.append(out.clone())
+        assert not torch.equal(out, eager[i])      # the eager call is split
+        assert_close(f32(out), f32(eager[i]), TOL_BF16, "unsplit")
+    outs, graphs = [torch.zeros_like(q) for q in qs], []
+    with RawStream() as st:
+        with torch.cuda.stream(st):
+            call(0, torch.empty_like(qs[0]))       # the stream's scratch
+        torch.cuda.synchronize()
+        for i in range(2):
+            graphs.append(torch.cuda.CUDAGraph())
+            with torch.cuda.graph(graphs[-1], stream=st):
+                call(i, outs[i])
+        torch.cuda.synchronize()
+        _replay_on_two_streams(graphs, outs, refs, "general prefill")
