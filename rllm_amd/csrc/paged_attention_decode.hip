@@ -1922,15 +1922,29 @@ int32_t mixed_impl(void* p_out, const void* p_q, const int32_t* p_bt, const int3
     const int64_t dpw = fp8 ? MIXED_DECODE_WAVES_FP8 : MIXED_DECODE_WAVES;
     const int max_waves = max_resident_waves();
     if (max_waves <= 0) return (int32_t)hipErrorInvalidDevice;
-    const int64_t nw = std::min<int64_t>(
-        max_waves, stream_waves(d_num_seqs, hkv, d_maxb, dpw * free_cus, 4 * free_cus, dpw <= 4));
-    const int64_t ws_bytes = nw > 1 ? stream_ws_bytes(max_waves, nw, G, d) : 0;
+    int64_t nw = 0, ws_bytes = 0;
+    auto plan_waves = [&](bool whole_rows) {
+        nw = std::min<int64_t>(
+            max_waves, stream_waves(d_num_seqs, hkv, d_maxb, dpw * free_cus, 4 * free_cus, dpw <= 4, whole_rows));
+        ws_bytes = nw > 1 ? stream_ws_bytes(max_waves, nw, G, d) : 0;
+    };
+    plan_waves(true);
     void* ws = nullptr;
     if (ws_bytes > 0) {
         // the arrival counters must start at zero (every call leaves them so)
-        const int32_t rc = g_workspaces.get(stream, WS_DECODE_STREAM, ws_bytes, true, &ws);
+        int32_t rc = g_workspaces.get(stream, WS_DECODE_STREAM, ws_bytes, true, &ws);
         if (rc) return rc;
-        if (!ws) return serial();   // capturing on a stream whose scratch is missing or too small
+        if (!ws) {
+            // capturing: scratch of a larger step may still hold equal shares
+            // (whole rows of 24 sequences want more waves than those of 25: 960
+            // against 800 on 200 CUs, FP8, 128-block tables)
+            plan_waves(false);
+            if (ws_bytes > 0) {
+                rc = g_workspaces.get(stream, WS_DECODE_STREAM, ws_bytes, true, &ws);
+                if (rc) return rc;
+                if (!ws) return serial();   // the stream's scratch is missing or too small
+            }
+        }
     }
     DecodeArgs da{};
     da.out = d_out;
