@@ -78,15 +78,28 @@ int64_t gen_scratch_bytes(const GenArgs& g) {
 
 // Library scratch of a split call; false and parts = 1 where there is none to be
 // had (a capture on a stream without it, no memory left).  `hold` keeps it until
-// the merge is queued.
-bool gen_take_scratch(GenArgs* g, hipStream_t stream, WorkspaceHold* hold) {
-    if (g->parts <= 1) return true;
+// the merge is queued.  `reserve` bytes are asked for first, by calls that do not
+// split too, so that a later capture finds them.
+bool gen_take_scratch(GenArgs* g, hipStream_t stream, WorkspaceHold* hold, int64_t reserve = 0) {
+    const bool split = g->parts > 1;
+    const int64_t need = split ? gen_scratch_bytes(*g) : 0;
+    const uintptr_t key = reinterpret_cast<uintptr_t>(stream);
     void* ws = nullptr;
-    const int32_t rc = g_workspaces.get(reinterpret_cast<uintptr_t>(stream), WS_GENERIC, gen_scratch_bytes(*g), false,
-                                        &ws, hold);
-    if (rc) (void)hipGetLastError();
-    return gen_set_scratch(g, rc ? nullptr : ws);
+    if (reserve > need && g_workspaces.get(key, WS_GENERIC, reserve, false, &ws, split ? hold : nullptr))
+        (void)hipGetLastError();
+    if (!split) return true;
+    if (!ws && g_workspaces.get(key, WS_GENERIC, need, false, &ws, hold)) (void)hipGetLastError();
+    return gen_set_scratch(g, ws);
 }
+
+// Units (workgroups of one part) and 512-token rounds of a decode, and the
+// workgroups that a split aims at: one or two fit a CU.
+int64_t gen_decode_units(const GenArgs& g) {
+    return static_cast<int64_t>(g.num_seqs) * g.hkv * ((g.hq / g.hkv + 15) / 16);
+}
+int64_t gen_decode_rounds(const GenArgs& g) { return (static_cast<int64_t>(g.maxb) * g.bs + 511) / 512; }
+int64_t gen_decode_want(const GenArgs& g, bool fp8) { return (g.d > 128 && !fp8 ? 2 : 4) * int64_t(gen_cus()); }
+constexpr int64_t GEN_MAX_PARTS = 64;   // gen_merge_kernel
 
 // Decode: parts of whole 512-token rounds (one window for each of a
 // workgroup's four waves), at most 64 (gen_merge_kernel), as many as give each
@@ -95,16 +108,28 @@ bool gen_take_scratch(GenArgs* g, hipStream_t stream, WorkspaceHold* hold) {
 // sequences of 4395 tokens, FP8, head_dim 128: 81.9 us at four rounds, 68.9
 // at two, 74.1 at one; 34 of 54-1742, head_dim 96: 44.0, 42.7, 47.3).
 void gen_decode_plan(GenArgs* g, bool fp8) {
-    const int64_t units = static_cast<int64_t>(g->num_seqs) * g->hkv * ((g->hq / g->hkv + 15) / 16);
-    const int64_t rounds = (static_cast<int64_t>(g->maxb) * g->bs + 511) / 512;
-    const int64_t want = (g->d > 128 && !fp8 ? 2 : 4) * int64_t(gen_cus());   // one or two workgroups fit a CU
-    int64_t parts = std::min<int64_t>(std::min<int64_t>(rounds, 64), (want + units - 1) / units);
+    const int64_t units = gen_decode_units(*g), rounds = gen_decode_rounds(*g), want = gen_decode_want(*g, fp8);
+    int64_t parts = std::min<int64_t>(std::min<int64_t>(rounds, GEN_MAX_PARTS), (want + units - 1) / units);
     if (parts < 1) parts = 1;
     const int64_t per = (rounds + parts - 1) / parts;
     g->chunk = static_cast<int32_t>(per * 512);
     g->parts = per > 0 ? static_cast<int32_t>((rounds + per - 1) / per) : 1;
     const int64_t slots = static_cast<int64_t>(g->rows) * g->hq * g->parts;
     if (units * g->parts > INT32_MAX || slots * (g->d + 2) > (int64_t(1) << 28)) g->parts = 1;
+}
+
+// Scratch for this call's table and any batch up to its own.  Large batches do
+// not split, small ones do: a program that warms up with its largest batch and
+// then captures the others would otherwise find nothing for them.  u units take
+// at most min(64, ceil(want / u)) parts, so at most want + u workgroups leave
+// partials (24/8 heads, head_dim 128: 3.2 MB; 16 heads a group: 17 MB).
+int64_t gen_decode_reserve(const GenArgs& g, bool fp8) {
+    const int64_t rounds = gen_decode_rounds(g);
+    if (rounds <= 1) return 0;
+    const int64_t units = gen_decode_units(g), want = gen_decode_want(g, fp8), G = g.hq / g.hkv;
+    const int64_t wgs = std::min(units * std::min<int64_t>(rounds, GEN_MAX_PARTS), want + std::min(units, want));
+    const int64_t heads = (G + (G + 15) / 16 - 1) / ((G + 15) / 16);   // of a unit, on average, rounded up
+    return wgs * heads * (g.d + 2) * 4;
 }
 
 // Prefill: few workgroups split the keys, at most 8 parts of at least 4
@@ -172,7 +197,7 @@ bool general_decode(void* out, const void* q, const void* kc, const void* vc, co
     if (!gen_mfma_shape(g, kv_dtype)) return false;
     gen_decode_plan(&g, fp8);
     WorkspaceHold hold;
-    if (!gen_take_scratch(&g, stream, &hold)) return false;
+    if (!gen_take_scratch(&g, stream, &hold, gen_decode_reserve(g, fp8))) return false;
     *rc = launch_gen_decode(g, q_dtype, kv_dtype, g.parts, stream);
     return true;
 }
@@ -200,7 +225,7 @@ int32_t generic_attention(void* out, const void* q, const void* kc, const void* 
         } else if (!may_allocate) {
             g.parts = 1;
         } else {
-            gen_take_scratch(&g, stream, &hold);
+            gen_take_scratch(&g, stream, &hold, gen_decode_reserve(g, fp8));
         }
         return launch_gen_decode(g, q_dtype, kv_dtype, g.parts, stream);
     }

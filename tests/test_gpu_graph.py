@@ -507,3 +507,42 @@ def test_mixed_step_captured_after_a_larger_one_stays_one_launch(dev):
             assert torch.equal(outs[0], eager[0]), f"replay {r}"
             assert_close(f32(outs[1]), f32(eager[1]), TOL_FP8, f"replay {r}")
             call(24, [torch.empty_like(pq), torch.empty_like(dq[:24])])
+
+
+@pytest.mark.parametrize("B", [8, 40])
+def test_general_decode_captured_after_a_larger_batch_is_split(dev, B):
+    """A batch of 128 fills the GPU without splitting its contexts, 40 and 8 do not.
+    The eager call of 128 leaves scratch for them: captured after it, they replay
+    the bits of their eager (split) calls."""
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(B)
+    rng = np.random.default_rng(B)
+    q = torch.randn((128, 24, 128), generator=gen, device=dev, dtype=torch.bfloat16)
+    kc, vc = (torch.randn((300, 8, 128, 32), generator=gen, device=dev, dtype=torch.bfloat16) for _ in range(2))
+    bt = ti(rng.integers(0, 300, (128, 128)).astype(np.int32), torch.int32, dev)
+    sl = ti(rng.integers(1, 4097, 128).astype(np.int32), torch.int32, dev)
+
+    def call(n, out, **kw):
+        return ops.paged_decode(q[:n], kc, vc, bt[:n], sl[:n], 0.1, out=out, validate=False, **kw)
+
+    log_case(f"general decode of {B} captured after 128")
+    eager = call(B, torch.empty_like(q[:B]))
+    unsplit = call(B, torch.empty_like(q[:B]), workspace=torch.zeros(16, dtype=torch.uint8, device=dev))
+    out = torch.zeros_like(eager)
+    torch.cuda.synchronize()
+    assert not torch.equal(eager, unsplit)
+    with RawStream() as st:
+        with torch.cuda.stream(st):
+            call(128, torch.empty_like(q))
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=st):
+            call(B, out)
+        for r in range(3):
+            out.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(st):
+                g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, eager), f"replay {r}"
+            call(B, torch.empty_like(eager))
