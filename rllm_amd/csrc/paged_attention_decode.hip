@@ -1614,7 +1614,7 @@ int32_t decode_impl(void* out, const void* q, const void* kc, const void* vc, co
         // a workspace sized for a larger call may fall short of whole rows (their
         // count does not always grow with the batch): equal shares then
         if (workspace && workspace_bytes < plan.ws_bytes) waves(false);
-        // without a caller's workspace short tables and few rows may run the
+        // without a caller's workspace few rows and short tables may run the
         // shape-general kernels.  The stream's scratch is reserved all the
         // same: a later capture of a smaller call may run the stream, and
         // cannot allocate it

@@ -158,30 +158,32 @@ GenArgs gen_args(void* out, const void* q, const void* kc, const void* vc, const
 }
 
 // Where the general decode beats the stream decode on the stream's own shapes
-// (block size 16, G = 1, 2, 4, 8).  Both take a few round trips for a short
-// call; the stream's grow with lengths that differ (its equal shares then cut
-// rows unevenly) and with the heads a wave carries, the general kernel's with
-// the rows (four waves each).  Kernel us, stream / general, head_dim 128,
-// sequences x tokens (a : b: lengths drawn from a to b):
-//   G = 4 (32/8 heads), up to 512 tokens.  8 x 1:100 14.2 / 10.7, 8 x 9:300 14.5
-//     / 12.0, 40 x 14:450 15.9 / 15.9; equal lengths 8 x 100 9.8 / 10.9, 8 x 300
-//     11.6 / 12.0, 64 x 320 20.6 / 17.9.  Tables of 8, 16, 24 or 32 blocks
-//     split evenly and stay, unless the rows are many: 40 x 128 10.3 / 12.0, 8 x
-//     512 11.8 / 13.7, 64 x 512 27.5 / 24.3; so does one sequence below 8
-//     blocks: 1 x 32 7.8 / 8.7.
-//   G = 4, long contexts of few rows: 1 x 12000 37.4 / 20.8, 1 x 24000 52.4 /
-//     29.9, 3 x 7000 27.3 / 26.3, 3 x 125:4000 29.7 / 18.7; kept: 1 x 4000 16.7 /
-//     18.2, 5 x 4000 22.8 / 25.8, 8 x 7000 40.5 / 48.2.
-//   G = 8 (32/4): 8 x 64 18.7 / 9.1, 8 x 512 15.8 / 13.5, 1 x 32768 99.8 / 25.2, 16
-//     x 4096 32.6 / 29.1; E4M3, head_dim 64: kept 64 x 4096 41.7 / 49.3.
+// (block size 16, G = 1, 2, 4, 8) whatever the lengths are: the call's plan knows
+// the table's width only.  Measured with full tables, lengths drawn from 1 to
+// the width, and tables ten times too wide; bf16 and E4M3, head_dim 64 and 128;
+// units = sequences x kv heads; the ratios are the slowest of the twelve, stream /
+// general.
+//   G = 8, one round of the general kernel (32 blocks): 1.06 at 512 units and
+//     1 block to 1.30 at 16; from 33 blocks the two-launch split costs more than it
+//     gives (0.84 - 0.97 at 33 to 64 blocks).
+//   G = 8, long tables of few units: the stream's 512-token shares are walked in
+//     series, the parts' windows by four waves each.  128 blocks 0.98 - 1.05, 200
+//     1.07 - 1.14, 256 1.12 - 1.22; 64 units 0.98 at 256 blocks, 0.96 at 400.
+//   G = 4, the same from 384 blocks (1.01 - 1.08; 300 blocks 0.90 - 0.94) up to 24
+//     units (24: 1.02 at 400, 1.10 at 500; 32: 0.95 - 0.98).  Shorter tables: 0.8
+//     - 1.1, faster only where lengths differ.
+//   Both end at 1024 tokens x units a CU (262144): one unit x 1000 blocks 2.0, x 16384 3.4
+//     (G = 4); past it 16 units 0.99 and 0.96 at 2048 and 4096 blocks, 8 units 1.02 at
+//     8192.
+// The lines stand for 256 CUs and move with their number.
 bool general_decode_pays(int64_t seqs, int64_t hkv, int64_t g, int64_t maxb) {
+    if (g != 4 && g != 8) return false;
     const int64_t units = seqs * hkv, tokens = maxb * 16;
-    if (units > 512) return false;
-    if (g >= 8) return maxb <= 32 || (tokens >= 4096 && units * tokens <= 262144);
-    if (g != 4) return false;
-    if (maxb <= 32) return maxb % 8 ? seqs > 1 || maxb > 8 : maxb >= 16 && units >= 500;
-    if (tokens >= 6144) return units * tokens <= 262144;
-    return tokens >= 3900 && units * tokens >= 40000 && units * tokens <= 131072;
+    const bool one_round = g == 8 && maxb <= 32;
+    if (!one_round && tokens < (g == 8 ? 4096 : 6144)) return false;
+    const int64_t cus = gen_cus();
+    if (one_round) return units <= 2 * cus;
+    return units * 32 <= cus * (g == 8 ? 4 : 3) && units * tokens <= 1024 * cus;
 }
 
 }  // namespace

@@ -1,6 +1,7 @@
-"""Decode of the stream kernel's own shapes where short tables or few rows run
-the shape-general kernels instead: both sides of every line of the rule, against
-the oracle and the stream (an explicit workspace always takes it)."""
+"""Decode of the stream kernel's own shapes where few long rows (GQA 4 and 8) or
+short tables (GQA 8) run the shape-general kernels instead: both sides of every
+line of the rule, tables wider than any context among them, against the oracle and
+the stream (an explicit workspace always takes it)."""
 import numpy as np
 import pytest
 import torch
@@ -19,14 +20,17 @@ CASES = [(1, 32, 8, 128, 7, O.BF16), (2, 32, 8, 128, 7, O.BF16), (1, 32, 8, 64, 
          (65, 32, 8, 128, 2, O.BF16), (64, 32, 8, 64, 16, O.FP8_E4M3), (62, 32, 8, 64, 16, O.FP8_E4M3),
          (9, 32, 8, 128, 31, O.BF16), (9, 32, 8, 128, 33, O.BF16), (1, 4, 1, 128, 384, O.BF16), (1, 4, 1, 128, 383, O.BF16),
          (5, 8, 2, 128, 250, O.BF16), (2, 32, 4, 64, 32, O.FP8_E5M2), (2, 32, 4, 64, 33, O.BF16),
-         (2, 8, 1, 128, 256, O.BF16), (3, 16, 8, 128, 7, O.BF16), (5, 8, 8, 64, 3, O.BF16)]
+         (2, 8, 1, 128, 256, O.BF16), (3, 16, 8, 128, 7, O.BF16), (5, 8, 8, 64, 3, O.BF16),
+         (128, 32, 4, 64, 3, O.BF16), (129, 32, 4, 64, 3, O.BF16), (2, 8, 1, 64, 255, O.FP8_E4M3),
+         (32, 8, 1, 64, 256, O.BF16), (33, 8, 1, 64, 256, O.BF16), (24, 4, 1, 64, 384, O.BF16),
+         (25, 4, 1, 64, 384, O.BF16), (1, 8, 1, 64, 16384, O.FP8_E5M2), (1, 8, 1, 64, 16385, O.FP8_E5M2)]
 
 
 @pytest.mark.parametrize("case", CASES, ids=[f"{c[0]}x{c[1]}:{c[2]}-D{c[3]}-{c[4]}blk-kv{c[5]}" for c in CASES])
 def test_both_routes_vs_oracle(dev, case):
     B, hq, hkv, d, maxb, kv = case
     rng = np.random.default_rng(B + maxb)
-    top = 16 * maxb
+    top = min(16 * maxb, 9000)               # past that: a table wider than its contexts
     q, k, v, bt, sl = random_case(rng, B, hq, hkv, d, (1 if B > 1 else top - 3, top), max_blocks=maxb, neg_blocks=1)
     if B > 2:
         sl[0], sl[1] = top, 0
