@@ -169,8 +169,9 @@ __device__ __forceinline__ int32_t clamp_pos(int32_t p, int32_t max_position) {
 // written as cache rows;
 // r >= Hkv: the q rotations of token r - Hkv (uniform position and cos / sin
 // row; lanes beyond Hq * D / 16 items idle).
-// RUNS: the kv part writes slot runs across the group's border; else whole rows only
-// where the 16 tokens are one run.
+// RUNS: the kv part writes slot runs across the group's border (block sizes with
+// 16-slot groups and aligned caches only); else whole rows only where the 16
+// tokens are one run.
 template <int IN_KIND, int CACHE_KIND, bool DIV, bool RNE, bool RUNS>
 __global__ __launch_bounds__(ROPE_THREADS) void rope_cache_kernel(
     uint16_t* q_out, const uint16_t* q, const uint16_t* __restrict__ k,
@@ -179,8 +180,9 @@ __global__ __launch_bounds__(ROPE_THREADS) void rope_cache_kernel(
     const float* __restrict__ cos_cache, const float* __restrict__ sin_cache, int64_t num_tokens,
     int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int64_t block_size,
     int64_t num_blocks, int32_t max_position, float k_scale, float v_scale, int32_t roles) {
-    extern __shared__ __align__(16) uint16_t lds[];   // [2][ROPE_STAGED][head_dim + 8]
-    __shared__ int64_t s_base[ROPE_STAGED];            // cache index of (token, head 0, d 0), or -1
+    constexpr int STAGED = RUNS ? ROPE_STAGED : ROPE_GROUP;
+    extern __shared__ __align__(16) uint16_t lds[];   // [2][STAGED][head_dim + 8]
+    __shared__ int64_t s_base[STAGED];                 // cache index of (token, head 0, d 0), or -1
     const int32_t role = static_cast<int32_t>(blockIdx.x % roles);
     const int64_t t0 = static_cast<int64_t>(blockIdx.x / roles) * ROPE_GROUP;
     const int32_t n_tok = static_cast<int32_t>(num_tokens - t0 < ROPE_GROUP ? num_tokens - t0 : ROPE_GROUP);
@@ -212,109 +214,17 @@ __global__ __launch_bounds__(ROPE_THREADS) void rope_cache_kernel(
         return;
     }
 
+    // lane i of each wave: the slot of token t0 - BACK + i, loaded before phase 1
+    // so that their round trip overlaps its loads
+    constexpr int BACK = RUNS ? 1 : 0, NSLOTS = RUNS ? 3 * ROPE_GROUP : ROPE_GROUP;
     const int32_t h = role;
-    if constexpr (!RUNS) {
-        // the group's slots, loaded before phase 1 so that their round trip
-        // overlaps its loads instead of following its LDS writes
-        int64_t sl = -1, s0 = -1;
-        if (threadIdx.x < ROPE_GROUP) {
-            s0 = slot_mapping[t0];
-            if (static_cast<int32_t>(threadIdx.x) < n_tok) sl = slot_mapping[t0 + threadIdx.x];
-        }
-        const int32_t stride = head_dim + 8;   // LDS row in elements (16-byte pad)
-        uint16_t* kl = lds;
-        uint16_t* vl = lds + ROPE_GROUP * stride;
-        const int64_t row_elems = static_cast<int64_t>(num_kv_heads) * head_dim;
-
-        // phase 1: rotated k and v rows of the group's tokens into LDS
-        const int32_t vit = head_dim >> 3;     // 16-byte items per row
-        for (int32_t it = threadIdx.x; it < n_tok * vit; it += ROPE_THREADS) {
-            const int32_t tok = it / vit;
-            const int32_t c = it - tok * vit;
-            const int64_t t = t0 + tok;
-            const int64_t row = (t * num_kv_heads + h) * head_dim;
-            *reinterpret_cast<uint4*>(vl + tok * stride + c * 8) = *reinterpret_cast<const uint4*>(v + row + c * 8);
-            if (c < per_head) {
-                const int32_t j0 = c * 8;
-                const int64_t pos = clamp_pos(positions[t], max_position);
-                uint4 o1, o2;
-                rotate8<IN_KIND>(k + row, j0, half, cos_cache + pos * half + j0, sin_cache + pos * half + j0,
-                                 o1, o2);
-                *reinterpret_cast<uint4*>(kl + tok * stride + j0) = o1;
-                *reinterpret_cast<uint4*>(kl + tok * stride + j0 + half) = o2;
-            }
-        }
-        // slots: padding (< 0) and blocks beyond the pool are skipped.  The rows go
-        // out as 16-element runs when the 16 tokens fill slots s0 .. s0+15 with s0
-        // a multiple of 16 inside one block (every prefill chunk), else per element.
-        int32_t run = 1;
-        if (threadIdx.x < ROPE_GROUP) {
-            const int32_t tok = threadIdx.x;
-            const int64_t blk = sl >= 0 ? sl / block_size : 0;
-            const bool valid = sl >= 0 && blk < num_blocks;
-            s_base[tok] = valid ? blk * row_elems * block_size + (sl - blk * block_size) : -1;
-            run = n_tok == ROPE_GROUP && block_size % ROPE_GROUP == 0 && s0 >= 0 && s0 % ROPE_GROUP == 0 &&
-                  sl == s0 + tok && valid &&
-                  ((reinterpret_cast<uintptr_t>(key_cache) | reinterpret_cast<uintptr_t>(value_cache)) & 15) == 0;
-        }
-        run = __syncthreads_and(run);
-
-        // phase 2: one (k or v, d) cache row per lane
-        for (int32_t r = threadIdx.x; r < 2 * head_dim; r += ROPE_THREADS) {
-            const bool is_v = r >= head_dim;
-            const int32_t d = is_v ? r - head_dim : r;
-            const uint16_t* col = (is_v ? vl : kl) + d;
-            void* cache = is_v ? value_cache : key_cache;
-            const float sc = is_v ? v_scale : k_scale;
-            const int64_t hd = (static_cast<int64_t>(h) * head_dim + d) * block_size;
-            if (run) {
-                uint16_t e[ROPE_GROUP];
-#pragma unroll
-                for (int tok = 0; tok < ROPE_GROUP; ++tok) e[tok] = col[tok * stride];
-                const int64_t idx = s_base[0] + hd;
-                if constexpr (CACHE_KIND == KIND_F16 || CACHE_KIND == KIND_BF16) {
-                    uint16_t lo[8], hi[8];
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        lo[i] = e[i];
-                        hi[i] = e[8 + i];
-                    }
-                    uint4* dst = reinterpret_cast<uint4*>(static_cast<uint16_t*>(cache) + idx);
-                    dst[0] = pack8(lo);
-                    dst[1] = pack8(hi);
-                } else {
-                    uint32_t w[4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        w[i] = static_cast<uint32_t>(enc8<IN_KIND, CACHE_KIND, DIV, RNE>(e[4 * i], sc)) |
-                               (static_cast<uint32_t>(enc8<IN_KIND, CACHE_KIND, DIV, RNE>(e[4 * i + 1], sc)) << 8) |
-                               (static_cast<uint32_t>(enc8<IN_KIND, CACHE_KIND, DIV, RNE>(e[4 * i + 2], sc)) << 16) |
-                               (static_cast<uint32_t>(enc8<IN_KIND, CACHE_KIND, DIV, RNE>(e[4 * i + 3], sc)) << 24);
-                    *reinterpret_cast<uint4*>(static_cast<uint8_t*>(cache) + idx) = make_uint4(w[0], w[1], w[2], w[3]);
-                }
-            } else {
-                for (int32_t tok = 0; tok < n_tok; ++tok) {
-                    const int64_t base = s_base[tok];
-                    if (base < 0) continue;
-                    const uint16_t x = col[tok * stride];
-                    if constexpr (CACHE_KIND == KIND_F16 || CACHE_KIND == KIND_BF16)
-                        static_cast<uint16_t*>(cache)[base + hd] = x;
-                    else
-                        static_cast<uint8_t*>(cache)[base + hd] = enc8<IN_KIND, CACHE_KIND, DIV, RNE>(x, sc);
-                }
-            }
-        }
-        return;
-    } else {
-    // lane i of each wave: the slot of token t0 - 1 + i (48 of them), loaded
-    // before phase 1 so that their round trip overlaps its loads
     const int32_t lane = static_cast<int32_t>(threadIdx.x & 63);
-    const int64_t ts = t0 - 1 + lane;
+    const int64_t ts = t0 - BACK + lane;
     int64_t slot = -1;
-    if (lane < 48 && ts >= 0 && ts < num_tokens) slot = slot_mapping[ts];
+    if (lane < NSLOTS && ts >= 0 && ts < num_tokens) slot = slot_mapping[ts];
     const int32_t stride = head_dim + 8;   // LDS row in elements (16-byte pad)
     uint16_t* kl = lds;
-    uint16_t* vl = lds + ROPE_STAGED * stride;
+    uint16_t* vl = lds + STAGED * stride;
     const int64_t row_elems = static_cast<int64_t>(num_kv_heads) * head_dim;
 
     // phase 1: rotated k and v rows of tokens t0 + [lo, hi) into LDS
@@ -339,28 +249,41 @@ __global__ __launch_bounds__(ROPE_THREADS) void rope_cache_kernel(
     };
     stage(0, n_tok);
 
-    // Slot runs: a run starts where a slot does not follow the one before it or
-    // opens a 16-slot group of a block; the workgroup writes the runs that start
-    // among its own tokens to their end (token 31 at most, which the next
-    // workgroup stages too), so a prompt that starts anywhere in the list still
-    // goes out as whole 16-slot rows.  Other block sizes and unaligned caches:
-    // every token is a run of its own.
-    const bool rows = block_size % ROPE_GROUP == 0 &&
-                      ((reinterpret_cast<uintptr_t>(key_cache) | reinterpret_cast<uintptr_t>(value_cache)) & 15) == 0;
-    const int64_t prev = (static_cast<int64_t>(__shfl_up(static_cast<int>(slot >> 32), 1)) << 32) |
-                         static_cast<uint32_t>(__shfl_up(static_cast<int>(slot), 1));
-    const bool start =
-        !rows || ts == 0 || ts >= num_tokens || slot < 0 || slot % ROPE_GROUP == 0 || slot != prev + 1;
-    const uint64_t starts = __builtin_amdgcn_ballot_w64(start && lane >= 1 && lane < 48) >> 1;
-    const uint64_t own = (uint64_t(1) << n_tok) - 1;
-    const uint64_t mine = starts & own;
-    if (!mine) return;   // whole workgroup: its tokens end a run of the one before
-    const int32_t end = __ffsll(static_cast<unsigned long long>(starts & ~own)) - 1;
-    if (end > n_tok) stage(n_tok, end);
+    // What the workgroup writes: tokens [first, stop) element by element, then, if
+    // `whole`, the 16 from `last` as rows.
+    int32_t first = 0, last = 0, stop;
+    bool whole;
+    if constexpr (RUNS) {
+        // A run starts where a slot does not follow the one before it or opens a
+        // 16-slot group of a block; the workgroup writes the runs that start among
+        // its own tokens to their end (token 31 at most, which the next workgroup
+        // stages too).  A run has at most 16 tokens, so only the last can fill a
+        // group.
+        const int64_t prev = (static_cast<int64_t>(__shfl_up(static_cast<int>(slot >> 32), 1)) << 32) |
+                             static_cast<uint32_t>(__shfl_up(static_cast<int>(slot), 1));
+        const bool start = ts == 0 || ts >= num_tokens || slot < 0 || slot % ROPE_GROUP == 0 || slot != prev + 1;
+        const uint64_t starts = __builtin_amdgcn_ballot_w64(start && lane >= 1 && lane < NSLOTS) >> 1;
+        const uint64_t own = (uint64_t(1) << n_tok) - 1, mine = starts & own;
+        if (!mine) return;   // whole workgroup: its tokens end a run of the one before
+        first = __ffsll(static_cast<unsigned long long>(mine)) - 1;
+        last = 63 - __builtin_clzll(mine);
+        const int32_t end = __ffsll(static_cast<unsigned long long>(starts & ~own)) - 1;
+        whole = end - last == ROPE_GROUP;
+        stop = whole ? last : end;
+        if (end > n_tok) stage(n_tok, end);
+    } else {
+        // rows where the 16 tokens fill slots s0 .. s0+15 of one group
+        const int64_t s0 = (static_cast<int64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(slot >> 32))) << 32) |
+                           static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(slot)));
+        whole = n_tok == ROPE_GROUP && block_size % ROPE_GROUP == 0 && s0 >= 0 && s0 % ROPE_GROUP == 0 &&
+                ((reinterpret_cast<uintptr_t>(key_cache) | reinterpret_cast<uintptr_t>(value_cache)) & 15) == 0 &&
+                !__builtin_amdgcn_ballot_w64(lane < ROPE_GROUP && slot != s0 + lane);
+        stop = whole ? 0 : n_tok;
+    }
     // where each token lands; padding (< 0) and blocks beyond the pool are skipped
-    if (threadIdx.x >= 1 && threadIdx.x <= ROPE_STAGED) {
+    if (threadIdx.x >= BACK && threadIdx.x < BACK + STAGED) {
         const int64_t blk = slot >= 0 ? slot / block_size : 0;
-        s_base[threadIdx.x - 1] =
+        s_base[threadIdx.x - BACK] =
             slot >= 0 && blk < num_blocks ? blk * row_elems * block_size + (slot - blk * block_size) : -1;
     }
     __syncthreads();
@@ -369,54 +292,44 @@ __global__ __launch_bounds__(ROPE_THREADS) void rope_cache_kernel(
     for (int32_t r = threadIdx.x; r < 2 * head_dim; r += ROPE_THREADS) {
         const bool is_v = r >= head_dim;
         const int32_t d = is_v ? r - head_dim : r;
+        const uint16_t* col = (is_v ? vl : kl) + d;
         void* cache = is_v ? value_cache : key_cache;
         const float sc = is_v ? v_scale : k_scale;
         const int64_t hd = (static_cast<int64_t>(h) * head_dim + d) * block_size;
-        for (uint64_t left = mine; left;) {
-            const int32_t a = __ffsll(static_cast<unsigned long long>(left)) - 1;
-            left &= left - 1;
-            const int32_t b = left ? __ffsll(static_cast<unsigned long long>(left)) - 1 : end;
-            const uint16_t* col = (is_v ? vl : kl) + a * stride + d;
-            if (b - a == ROPE_GROUP) {
-                const int64_t base = s_base[a];
-                if (base < 0) continue;
-                uint16_t e[ROPE_GROUP];
-#pragma unroll
-                for (int tok = 0; tok < ROPE_GROUP; ++tok) e[tok] = col[tok * stride];
-                const int64_t idx = base + hd;
-                if constexpr (CACHE_KIND == KIND_F16 || CACHE_KIND == KIND_BF16) {
-                    uint16_t lo[8], hi[8];
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        lo[i] = e[i];
-                        hi[i] = e[8 + i];
-                    }
-                    uint4* dst = reinterpret_cast<uint4*>(static_cast<uint16_t*>(cache) + idx);
-                    dst[0] = pack8(lo);
-                    dst[1] = pack8(hi);
-                } else {
-                    uint32_t w[4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        w[i] = static_cast<uint32_t>(enc8<IN_KIND, CACHE_KIND, DIV, RNE>(e[4 * i], sc)) |
-                               (static_cast<uint32_t>(enc8<IN_KIND, CACHE_KIND, DIV, RNE>(e[4 * i + 1], sc)) << 8) |
-                               (static_cast<uint32_t>(enc8<IN_KIND, CACHE_KIND, DIV, RNE>(e[4 * i + 2], sc)) << 16) |
-                               (static_cast<uint32_t>(enc8<IN_KIND, CACHE_KIND, DIV, RNE>(e[4 * i + 3], sc)) << 24);
-                    *reinterpret_cast<uint4*>(static_cast<uint8_t*>(cache) + idx) = make_uint4(w[0], w[1], w[2], w[3]);
-                }
-            } else {
-                for (int32_t tok = a; tok < b; ++tok) {
-                    const int64_t base = s_base[tok];
-                    if (base < 0) continue;
-                    const uint16_t x = col[(tok - a) * stride];
-                    if constexpr (CACHE_KIND == KIND_F16 || CACHE_KIND == KIND_BF16)
-                        static_cast<uint16_t*>(cache)[base + hd] = x;
-                    else
-                        static_cast<uint8_t*>(cache)[base + hd] = enc8<IN_KIND, CACHE_KIND, DIV, RNE>(x, sc);
-                }
-            }
+        for (int32_t tok = first; tok < stop; ++tok) {
+            const int64_t base = s_base[tok];
+            if (base < 0) continue;
+            const uint16_t x = col[tok * stride];
+            if constexpr (CACHE_KIND == KIND_F16 || CACHE_KIND == KIND_BF16)
+                static_cast<uint16_t*>(cache)[base + hd] = x;
+            else
+                static_cast<uint8_t*>(cache)[base + hd] = enc8<IN_KIND, CACHE_KIND, DIV, RNE>(x, sc);
         }
-    }
+        if (!whole || s_base[last] < 0) continue;
+        uint16_t e[ROPE_GROUP];
+#pragma unroll
+        for (int tok = 0; tok < ROPE_GROUP; ++tok) e[tok] = col[(last + tok) * stride];
+        const int64_t idx = s_base[last] + hd;
+        if constexpr (CACHE_KIND == KIND_F16 || CACHE_KIND == KIND_BF16) {
+            uint16_t lo[8], hi[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                lo[i] = e[i];
+                hi[i] = e[8 + i];
+            }
+            uint4* dst = reinterpret_cast<uint4*>(static_cast<uint16_t*>(cache) + idx);
+            dst[0] = pack8(lo);
+            dst[1] = pack8(hi);
+        } else {
+            uint32_t w[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                w[i] = static_cast<uint32_t>(enc8<IN_KIND, CACHE_KIND, DIV, RNE>(e[4 * i], sc)) |
+                       (static_cast<uint32_t>(enc8<IN_KIND, CACHE_KIND, DIV, RNE>(e[4 * i + 1], sc)) << 8) |
+                       (static_cast<uint32_t>(enc8<IN_KIND, CACHE_KIND, DIV, RNE>(e[4 * i + 2], sc)) << 16) |
+                       (static_cast<uint32_t>(enc8<IN_KIND, CACHE_KIND, DIV, RNE>(e[4 * i + 3], sc)) << 24);
+            *reinterpret_cast<uint4*>(static_cast<uint8_t*>(cache) + idx) = make_uint4(w[0], w[1], w[2], w[3]);
+        }
     }
 }
 
@@ -457,7 +370,7 @@ constexpr int64_t ROPE_RUNS_MIN = 384;
 template <int IN_KIND, int CACHE_KIND, bool RNE = false>
 int32_t launch_rope(dim3 grid, hipStream_t st, const RopeArgs& a) {
     constexpr bool fp8 = CACHE_KIND == KIND_FP8_E4M3 || CACHE_KIND == KIND_FP8_E5M2;
-    const bool runs = a.n >= ROPE_RUNS_MIN;
+    const bool runs = a.n >= ROPE_RUNS_MIN && a.bs % ROPE_GROUP == 0 && aligned16(a.kc) && aligned16(a.vc);
     const size_t lds = 2u * (runs ? ROPE_STAGED : ROPE_GROUP) * (a.d + 8) * sizeof(uint16_t);
     const bool div = fp8 && !(pow2(a.ks) && pow2(a.vs));
     const float ks = div ? a.ks : fp8 ? 1.0f / a.ks : 1.0f, vs = div ? a.vs : fp8 ? 1.0f / a.vs : 1.0f;
