@@ -22,7 +22,7 @@
 // One token's column touches every row of its tiles, so each byte (FP8) or
 // 16-bit element stored costs a separate write of a whole memory sector; the
 // layout fixes that for single-token writes.  Longer token lists, prompts among
-// them, run cache_write_runs_kernel.
+// them, run cache_write_runs_kernel (RUNS_ELEMS).
 #include "common.h"
 #include "../../include/rllm_kernels.h"
 
@@ -267,13 +267,17 @@ int32_t validate_write(const void* kc, const void* vc, const void* nk, const voi
     return 0;
 }
 
-// Tokens from which cache_write_runs_kernel takes a call: below, a batch of
-// decode tokens (no runs) is faster one token a workgroup.  8 x 128 elements a
-// token, kernel us, one token a workgroup / runs: 256 decode tokens bf16 7.4 /
-// 7.5, E4M3 6.3 / 7.1; a prompt of 200 5.6 / 3.6; 2 of 256 9.6 / 3.6, E4M3 8.7
-// / 5.2; 8 of 512 44.6 / 8.9, 43.0 / 12.7.  From 2048 tokens 128 elements a
-// workgroup instead of 64: 44.6 / 8.7, 43.0 / 10.8.
-constexpr int64_t RUNS_MIN = 384, RUNS_WIDE = 2048;
+// Whether cache_write_runs_kernel takes a call: its tokens times row elements (a
+// token's k or v) decide, as they fill the chip; below, a batch of decode tokens
+// (no runs) is faster one token a workgroup.  Kernel us, one token a workgroup /
+// runs, at the line of 393216 elements: decode tokens of 32, 16, 8 and 2 x 128 bf16
+// 12.4 / 10.1, 11.0 / 9.5, 10.2 / 9.5, 9.8 / 9.4, E4M3 10.8 / 8.9, 9.7 / 8.9, 9.1 / 9.0, 8.9 /
+// 9.0; one prompt 9.0 / 4.3, E4M3 8.3 / 5.8.  At 294912: 8 x 128 9.3 / 8.8, E4M3 8.2 /
+// 8.3, 2 x 128 8.6 / 8.8, 7.5 / 8.4; a prompt of 200 tokens of 8 x 128 5.6 / 3.6.  Rows
+// of 128 elements later: 3072 decode tokens 9.9 / 9.6, E4M3 9.1 / 9.6, 4096 11.4 /
+// 10.9, 10.9 / 10.3.  From 2048 tokens 128 elements a workgroup instead of 64 (4096 of 8 x 128:
+// 8.9 -> 8.7, E4M3 12.7 -> 10.8).
+constexpr int64_t RUNS_ELEMS = 393216, RUNS_ELEMS_NARROW = 524288, RUNS_WIDE = 2048;
 
 template <int CACHE_KIND, bool RNE = false>
 int32_t launch_write(void* kc, void* vc, const uint16_t* nk, const uint16_t* nv, const int64_t* sm,
@@ -294,8 +298,9 @@ int32_t launch_write(void* kc, void* vc, const uint16_t* nk, const uint16_t* nv,
     }
     const uintptr_t ptrs = reinterpret_cast<uintptr_t>(kc) | reinterpret_cast<uintptr_t>(vc) |
                            reinterpret_cast<uintptr_t>(nk) | reinterpret_cast<uintptr_t>(nv);
-    const bool runs = n >= RUNS_MIN && bs % 16 == 0 && (hkv * d) % 8 == 0 && ptrs % 16 == 0 &&
-                      (n + 15) / 16 * ((hkv * d + 63) / 64) <= INT32_MAX;
+    const int64_t row = hkv * d;
+    const bool runs = n * row >= (row < 256 ? RUNS_ELEMS_NARROW : RUNS_ELEMS) && bs % 16 == 0 && row % 8 == 0 &&
+                      ptrs % 16 == 0 && (n + 15) / 16 * ((row + 63) / 64) <= INT32_MAX;
     auto go = [&](auto div_tag) {
         constexpr bool DIV = decltype(div_tag)::value;
         const float ks = DIV ? k_scale : (fp8 ? 1.0f / k_scale : 1.0f);

@@ -27,9 +27,8 @@
 // (token, row).  A workgroup writes the runs that start among its 16 tokens, to
 // their end: prompts that start anywhere in the list go out as whole rows (6
 // prompts, 3152 tokens of 32/8 heads, head_dim 128, through the torch front end:
-// 25.3 us with whole rows only where the 16 tokens are one run, 15.8 so; E4M3
-// 19.1, 18.4; 8 of 512, all aligned, 21.0 both); short calls stay with their own
-// group (ROPE_RUNS_MIN).  One workgroup per token
+// 25.3 us with whole rows only where the 16 tokens are one run, 15.8 so); short
+// calls stay with their own group (ROPE_RUNS_ELEMS).  One workgroup per token
 // rotates q into q_out (16-byte loads and stores, in place allowed).  A
 // rotation item is 8 elements of the first half of a head and their 8 partners
 // in the second half; bf16 rounding uses the packed hardware conversion
@@ -361,16 +360,27 @@ struct RopeArgs {
     int32_t roles;
 };
 
-// Tokens from which the kv part follows slot runs: a batch of decode tokens has
-// none and is faster without the search.  32/8 heads, head_dim 128, kernel us,
-// without / with: 64 decode tokens 6.6 / 7.0, 256 8.7 / 9.2, E4M3 8.7 / 9.8; 6
-// prompts, 3152 tokens, 25.4 / 16.1, E4M3 19.1 / 18.5.
-constexpr int64_t ROPE_RUNS_MIN = 384;
+// Whether the kv part follows slot runs: the call's tokens times row elements (a
+// token's k or v) decide, as they fill the chip.  The list may be decode tokens,
+// prompts that start anywhere or one aligned prompt; kernel us without / with
+// runs, at rows of 512 to 4096 elements, head_dim 64 and 128:
+//   bf16, 2^19 elements (512 tokens of 8 x 128): decode 13.4 / 13.5, one prompt 6.7
+//     / 6.8, four unaligned prompts 8.6 / 8.7, half of each 10.8 / 10.5; of 16 x 128 9.6 /
+//     8.2 unaligned.  2^20: 27.7 / 27.6, 8.7 / 8.8, 12.0 / 10.7, 17.4 / 17.2; 2^22: 110 / 110,
+//     23.8 / 23.8, 38.2 / 26.0, 72.1 / 66.0.  Below: 192 tokens of 8 x 128 unaligned 6.6 /
+//     7.0 (a second round trip for the tokens past the group)
+//   FP8 (encoding beside it), 2^21: 29.1 / 29.5, 14.7 / 15.0, 17.5 / 17.5, 24.8 / 24.2; 2^22:
+//     49.6 / 49.7, 23.9 / 24.1, 29.1 / 27.1; 2^20: unaligned 10.9 / 12.0
+// Narrower rows leave few kv workgroups, whose search then shows: 3072 tokens of 2
+// x 128 decode 17.1 / 18.0, one prompt 8.3 / 8.9.
+constexpr int64_t ROPE_RUNS_ELEMS = 1 << 19, ROPE_RUNS_ELEMS_FP8 = 1 << 21, ROPE_RUNS_ROW = 512;
 
 template <int IN_KIND, int CACHE_KIND, bool RNE = false>
 int32_t launch_rope(dim3 grid, hipStream_t st, const RopeArgs& a) {
     constexpr bool fp8 = CACHE_KIND == KIND_FP8_E4M3 || CACHE_KIND == KIND_FP8_E5M2;
-    const bool runs = a.n >= ROPE_RUNS_MIN && a.bs % ROPE_GROUP == 0 && aligned16(a.kc) && aligned16(a.vc);
+    const int64_t row = static_cast<int64_t>(a.hkv) * a.d;
+    const bool runs = row >= ROPE_RUNS_ROW && a.n * row >= (fp8 ? ROPE_RUNS_ELEMS_FP8 : ROPE_RUNS_ELEMS) &&
+                      a.bs % ROPE_GROUP == 0 && aligned16(a.kc) && aligned16(a.vc);
     const size_t lds = 2u * (runs ? ROPE_STAGED : ROPE_GROUP) * (a.d + 8) * sizeof(uint16_t);
     const bool div = fp8 && !(pow2(a.ks) && pow2(a.vs));
     const float ks = div ? a.ks : fp8 ? 1.0f / a.ks : 1.0f, vs = div ? a.vs : fp8 ? 1.0f / a.vs : 1.0f;

@@ -31,9 +31,11 @@ def _slots(rng, n, bs):
     return out, nb - 1               # ids nb - 1 and nb lie past the pool
 
 
-# (kv heads, head_dim, block size, tokens)
+# (kv heads, head_dim, block size, tokens): slot runs from 393216 elements (rows below
+# 256 elements: 524288), 64 of them a workgroup, 128 from 2048 tokens
 SHAPES = [(8, 128, 16, 384), (8, 128, 16, 385), (8, 128, 32, 2047), (8, 128, 16, 2049), (1, 40, 48, 700),
-          (3, 24, 16, 2500), (1, 8, 64, 399)]
+          (3, 24, 16, 2500), (1, 8, 64, 399), (8, 128, 16, 383), (32, 128, 16, 97), (1, 264, 32, 1500),
+          (2, 96, 48, 2729), (2, 96, 48, 2735), (1, 40, 48, 13111), (3, 24, 16, 7300)]
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=[f"{s[0]}x{s[1]}-bs{s[2]}-n{s[3]}" for s in SHAPES])
@@ -70,7 +72,7 @@ def test_cache_write_runs_bit_exact(dev, shape, cache):
 
 def test_cache_write_unaligned_rows_take_the_token_kernel(dev):
     # rows two bytes past a 16-byte boundary: the same bytes
-    hkv, d, bs, n = 2, 64, 16, 500
+    hkv, d, bs, n = 4, 64, 16, 1600
     rng = np.random.default_rng(4)
     sl, nb = _slots(rng, n, bs)
     nk = O.encode(rng.standard_normal((n, hkv, d)).astype(np.float32), O.F16)
@@ -88,13 +90,41 @@ def test_cache_write_unaligned_rows_take_the_token_kernel(dev):
 
 
 # (kv heads, head_dim, block size, tokens): whole and part groups, one token past a
-# group, a block size without 16-slot groups, the widest head
+# group, a block size without 16-slot groups, the widest head; each list within the
+# workgroups' own groups (short) and, from 2^19 elements, 2^21 of an FP8 cache, in slot
+# runs across them
 ROPE_SHAPES = [(8, 128, 16, 384), (2, 64, 32, 433), (1, 16, 16, 31), (1, 96, 16, 17), (2, 80, 24, 100), (1, 512, 16, 150)]
+ROPE_LONG = [(8, 128, 16, 512), (8, 64, 32, 1039), (32, 16, 16, 1025), (6, 96, 16, 913), (1, 512, 16, 1031),
+             (8, 80, 24, 900), (8, 128, 16, 511), (2, 128, 16, 2100)]
 
 
-@pytest.mark.parametrize("shape", ROPE_SHAPES, ids=[f"{s[0]}x{s[1]}-bs{s[2]}-n{s[3]}" for s in ROPE_SHAPES])
+@pytest.mark.parametrize("shape", ROPE_SHAPES + ROPE_LONG,
+                         ids=[f"{s[0]}x{s[1]}-bs{s[2]}-n{s[3]}" for s in ROPE_SHAPES + ROPE_LONG])
 @pytest.mark.parametrize("cache", [O.BF16, O.FP8_E4M3, O.FP8_E5M2])
 def test_rope_cache_runs_bit_exact(dev, shape, cache):
     hkv, d, bs, n = shape
+    if shape in ROPE_LONG and cache != O.BF16:
+        n = 4 * n + (n & 1)
     sl, nb = _slots(np.random.default_rng(n + d), n, bs)
     rope_run(dev, n, 2 * hkv, hkv, d, nb, bs, O.BF16, cache, slots=sl, ks=0.5, vs=0.37, rne=cache == O.FP8_E5M2)
+
+
+def test_rope_unaligned_cache_is_written_element_by_element(dev):
+    # caches two elements past a 16-byte boundary, a list long enough for runs
+    n, hkv, d, bs = 700, 8, 128, 16
+    rng = np.random.default_rng(12)
+    sl, nb = _slots(rng, n, bs)
+    k, v = (O.encode(rng.standard_normal((n, hkv, d)).astype(np.float32), O.BF16) for _ in range(2))
+    kd, vd = t16(k, torch.bfloat16, dev), t16(v, torch.bfloat16, dev)
+    pos = ti(rng.integers(0, 512, n).astype(np.int32), torch.int32, dev)
+    cos, sin = ops.rope_cache_tables(512, d, 10000.0, device=dev)
+    size = nb * hkv * d * bs
+    flat = [torch.zeros(size + 2, dtype=torch.bfloat16, device=dev) for _ in range(2)]
+    odd = [f[2:].view(nb, hkv, d, bs) for f in flat]
+    even = [torch.zeros((nb, hkv, d, bs), dtype=torch.bfloat16, device=dev) for _ in range(2)]
+    log_case("rope, unaligned caches")
+    for kc, vc in (odd, even):
+        ops.rope_and_cache(None, kd, vd, kc, vc, ti(sl, torch.int64, dev), pos, cos, sin)
+    torch.cuda.synchronize()
+    for a, b in zip(odd, even):
+        assert np.array_equal(bits16(a), bits16(b)) and b.any()
