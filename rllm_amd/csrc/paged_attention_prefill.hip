@@ -194,11 +194,12 @@ int32_t prefill_impl(void* out, const void* q, const void* kc, const void* vc, c
     const int64_t splits = chunk_splits(nwg, maxb);
     a.splits = static_cast<int32_t>(splits);
     a.base_wgs = static_cast<int32_t>(nwg);
-    // more workgroups than CUs: the longest tiles first (5 prompts of 1459 fresh
-    // tokens, 16/4 heads: 74.6 us sequence by sequence, 58.2 so; 8 of 512 on
-    // 2048: 147.7, 143.9; 6 of 237-1541: 83.6, 86.6).  A single round keeps the
-    // cheaper lookup.
-    a.longest_first = splits == 1 && nwg > device_cu_count() && num_seqs <= LONGEST_MAX_SEQS;
+    // the workgroups are more than one and at most two rounds, as far as the host
+    // can tell (nwg is the most there can be): the kernel counts them
+    const int64_t cus = device_cu_count(), qt = PP_ROWS / G;
+    if (splits == 1 && G >= 4 && num_seqs >= LONGEST_MIN_SEQS && num_seqs <= LONGEST_MAX_SEQS && nwg > cus &&
+        (num_tokens + qt - 1) / qt * hkv <= 2 * cus)
+        a.longest_cus = static_cast<int32_t>(cus);
     const int64_t rows = num_tokens * hq;
     int64_t splits_used = splits;
     WorkspaceHold hold;   // until the merge is queued

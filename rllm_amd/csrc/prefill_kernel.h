@@ -15,7 +15,7 @@
 //               every K/V tile staged in LDS serves the whole group.  One
 //               workgroup per CU, two waves per SIMD.  A sequence's last
 //               query tile (the most keys) is launched first, or, in a
-//               grid of several rounds, the batch's tiles by falling key
+//               grid of one to two rounds, the batch's tiles by falling key
 //               counts, so the workgroups that start later are the short ones.
 //   KV tile   = 64 tokens (four cache blocks) in LDS in the cache's own
 //               layout ([block][d][16 tokens]), three buffers.
@@ -133,12 +133,21 @@ struct PrefillArgs {
     // block_tables[0] (max_blocks = the prefix's blocks), and every row of
     // the batch writes a partial, also with one split
     int32_t prefix_tokens, prefix_queries;
-    // query tiles in the order of falling key counts over all sequences
-    // (longest_tile) instead of sequence by sequence; at most LONGEST_MAX_SEQS
-    int32_t longest_first;
+    // the device's CUs where the batch may take its query tiles by falling key
+    // counts over all sequences (longest_tile), 0: sequence by sequence
+    int32_t longest_cus;
 };
 
-constexpr int LONGEST_MAX_SEQS = 16;
+// Tiles by falling key counts: 3 to 12 sequences, GQA 4 or 8, and more than 17/16
+// and at most 2 workgroups a CU, counted by the kernel from the lengths themselves.
+// The second round is then partly filled, and the short tiles fill it.  178
+// random batches (8/2, 16/4, 32/8, 32/4 heads, equal and uneven, fresh and cached):
+// 1.09 times as fast on average, 144 faster by over 1.5%, 4 slower by that (1.6 - 3.4%);
+// 5 x 1024 fresh tokens, 16/4 heads, 53.7 -> 37.2 us, 8 x 512 on 2048, 32/8, 149.4 -> 145.2.  With
+// more rounds the order mixes the sequences' keys for less: 16 x 512, 32/8, 80.1 ->
+// 82.5, 6 x 237-1541 83.6 -> 86.6; GQA 1 and 2 as often slower as faster; 13 to 16
+// sequences of few tiles pay the longer lookup (27.9 -> 30.6).
+constexpr int LONGEST_MIN_SEQS = 3, LONGEST_MAX_SEQS = 12;
 
 // Transposing LDS read: in each group of 16 lanes, lane j addresses 4
 // consecutive 16-bit values M[j][0..3]; lane i receives M[4k + i/4][i%4]
@@ -319,12 +328,14 @@ __device__ __forceinline__ void prefill_body(PrefillArgs a, const int32_t* __res
             n_l = a.query_start_loc[lane + 1] - q0_l;
             ctx_l = a.seq_lens[lane];
         }
-        if (a.longest_first) {
+        const int nt_l = n_l > 0 ? (n_l + QT - 1) / QT : 0;
+        const int incl_l = seq_scan(nt_l);
+        const int wgs = __builtin_amdgcn_readlane(incl_l, 63) * a.num_kv_heads;
+        if (wgs > a.longest_cus + a.longest_cus / 16 && wgs <= 2 * a.longest_cus) {
             s = longest_tile<QT>(a.num_seqs, lane, n_l, ctx_l, j, tile);
             if (s < 0) return;                // whole workgroup: no barrier is reached
         } else {
-            const int nt_l = n_l > 0 ? (n_l + QT - 1) / QT : 0;
-            const int first_l = seq_scan(nt_l) - nt_l;
+            const int first_l = incl_l - nt_l;
             const uint64_t hit = __builtin_amdgcn_ballot_w64(first_l <= j && j < first_l + nt_l);
             if (!hit) return;                 // whole workgroup
             s = __ffsll(static_cast<unsigned long long>(hit)) - 1;
