@@ -38,6 +38,11 @@
  * any non-null one, however small, keeps the library's scratch out).
  * Cache writes accept any shape.
  *
+ * Alignment in bytes for the tuned attention kernels: caches 16 (FP8: 8), prefill
+ * queries 16 and outputs 8, decode queries 4 and outputs 2.  The shape-general
+ * kernels take any; queries, outputs or caches short of 16 (FP8 caches: 8) leave
+ * the matrix cores out.
+ *
  * Differences from the reference kernels, all deliberate:
  *   - a sequence with seq_len <= 0 gets an all-zero output row (the reference
  *     leaves it unwritten, paged_attention.cu:110);

@@ -838,7 +838,9 @@ __device__ __forceinline__ void prefill_body(PrefillArgs a, const int32_t* __res
         return;
     }
     // lanes l and l + 32 hold the two halves of each 16-byte run; swapped in
-    // pairs of runs, lane l stores the whole run 2r and lane l + 32 run 2r + 1
+    // pairs of runs, lane l stores the whole run 2r and lane l + 32 run 2r + 1.
+    // The output may be a view that starts on an 8-byte boundary.
+    typedef uint32_t out_run __attribute__((ext_vector_type(4), aligned(8)));
     const float inv = l > 0.f ? a.v_scale / l : 0.f;
     uint16_t* dst = static_cast<uint16_t*>(a.out) + orow * D + 8 * hl;
 #pragma unroll
@@ -855,7 +857,7 @@ __device__ __forceinline__ void prefill_body(PrefillArgs a, const int32_t* __res
                 w[i] = r[0];
                 w[2 + i] = r[1];
             }
-            *reinterpret_cast<uint4*>(dst + 32 * dt + 8 * jj) = make_uint4(w[0], w[1], w[2], w[3]);
+            *reinterpret_cast<out_run*>(dst + 32 * dt + 8 * jj) = out_run{w[0], w[1], w[2], w[3]};
         }
 }
 

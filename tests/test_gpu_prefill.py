@@ -358,3 +358,31 @@ def test_prefill_kv_split_merge_is_deterministic(dev):
     assert_close(runs[0], ref, TOL_BF16, "kv split determinism vs oracle")
     for i in range(1, 4):
         assert np.array_equal(runs[i], runs[0]), f"run {i} differs from run 0"
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_prefill_output_on_an_8_byte_boundary(dev, D, mixed):
+    """A contiguous output view that starts 4 elements into its buffer gets the
+    bits of an aligned one, and nothing around it changes."""
+    rng = np.random.default_rng(93)
+    hq, hkv = 32, 8
+    q, k, v, bt, sl, qsl = make_case(rng, [130, 1, 70], [40, 0, 300], hq, hkv, D)
+    bf = torch.bfloat16
+    dq, kc, vc = (t16(O.encode(x, O.BF16), bf, dev) for x in (q, k, v))
+    dbt, dsl, dqsl = ti(bt, torch.int32, dev), ti(sl, torch.int32, dev), ti(qsl, torch.int32, dev)
+
+    def call(out):
+        if not mixed:
+            return ops.paged_prefill(dq, kc, vc, dbt, dsl, dqsl, 0.1, out=out, validate=False)
+        ops.paged_mixed(dq, dbt, dsl, dqsl, dq[:3].contiguous(), dbt, dsl, kc, vc, 0.1, prefill_out=out, validate=False)
+        return out
+
+    log_case(f"prefill output 8 bytes off D={D} mixed={mixed}")
+    ref = call(torch.empty_like(dq))
+    buf = torch.full((dq.numel() + 8,), 7.0, dtype=bf, device=dev)
+    out = call(buf[4:4 + dq.numel()].view(dq.shape))
+    torch.cuda.synchronize()
+    assert out.data_ptr() % 16 == 8
+    assert torch.equal(out, ref)
+    assert (buf[:4] == 7).all() and (buf[-4:] == 7).all()
