@@ -179,7 +179,7 @@ struct DecodeArgs {
     int32_t num_seqs, num_q_heads, num_kv_heads, max_blocks;
     int32_t part_chunks;   // partitioned mode: 512-token super-chunks per partition
     int32_t max_parts;
-    int32_t num_waves;     // stream mode: waves (= workgroups) in the grid
+    int32_t num_waves;     // stream mode: waves in the grid, and shares of a batch of equal lengths
     float s_scale;         // scale * log2(e) * k_scale
     float v_scale;
     // cascade over a shared prefix (partitioned mode; 0 otherwise): the
@@ -188,6 +188,10 @@ struct DecodeArgs {
     // slots of a row hold the prefix partials) and every row is reduced
     int32_t block_offset;
     int32_t part_offset;
+    // stream: shares of a batch of mixed lengths, at most num_waves.  Last, past what the
+    // kernels load in one piece: beside num_waves it spilled scalar registers in one
+    // instantiation (32/16 heads, D 64: 9.6 -> 10.0 us at 3 x 16-48 tokens)
+    int32_t mixed_waves;
 };
 
 __device__ __forceinline__ int num_parts_for(int ctx_blocks, int part_chunks) {
@@ -1177,7 +1181,8 @@ __device__ __forceinline__ void decode_stream_body(const DecodeArgs& a, typename
     // items span, so there are at most as many shares as items (the grid is
     // sized from the table width, which can exceed the contexts by far).  A
     // share of virtual items only has no piece and lies in no row's count.
-    const int nws = static_cast<int>(min(static_cast<int64_t>(nw), total));
+    const int shares = ROW_COST > 0 ? a.mixed_waves : nw;   // mixed lengths : equal ones
+    const int nws = static_cast<int>(min(static_cast<int64_t>(shares), total));
     if (w >= nws) return;
     const WorkList wl{total, nws};
     const int64_t lo = wl.share_begin(w);
@@ -1378,7 +1383,7 @@ struct Plan {
     Mode mode = Mode::Stream;
     int32_t part_chunks = 0;
     int32_t max_parts = 0;
-    int32_t num_waves = 0;
+    int32_t num_waves = 0, mixed_waves = 0;
     int32_t max_waves = 0;   // stream mode: device bound on resident waves
     int64_t ws_bytes = 0;
 };
@@ -1418,6 +1423,11 @@ int max_resident_waves() {
     return cus * (thr / 64);
 }
 
+struct StreamWaves {
+    int64_t waves;   // the grid's, and a batch of equal lengths' shares
+    int64_t mixed;   // shares of a batch of mixed lengths, which the kernel tells apart
+};
+
 // simds: SIMDs of the device (4 per CU; 0 if unknown: then half the
 // resident bound stands in for it).
 // one_per_simd: 16-bit caches stop at one wave per SIMD and give each wave
@@ -1429,9 +1439,9 @@ int max_resident_waves() {
 // 233.8 us at one per SIMD).
 // whole_rows: false gives the equal shares that ignore row ends, never more waves
 // than whole rows.
-int64_t stream_waves(int64_t num_seqs, int64_t hkv, int64_t max_blocks, int64_t resident,
-                     int64_t simds, bool one_per_simd, bool whole_rows = true) {
-    const int64_t work_bound = num_seqs * hkv * max_blocks;
+StreamWaves stream_waves(int64_t num_seqs, int64_t hkv, int64_t max_blocks, int64_t resident,
+                         int64_t simds, bool one_per_simd, bool whole_rows = true) {
+    const int64_t rows = num_seqs * hkv, work_bound = rows * max_blocks;
     int64_t per_wave =
         std::min(STREAM_BLOCKS_PER_WAVE_MAX, std::max(STREAM_BLOCKS_PER_WAVE_MIN, max_blocks / 4));
     // at least one wave per SIMD where the table holds enough work: a small
@@ -1440,16 +1450,26 @@ int64_t stream_waves(int64_t num_seqs, int64_t hkv, int64_t max_blocks, int64_t 
     if (per_simd > 0)
         per_wave = std::min(per_wave,
                             std::max(STREAM_BLOCKS_PER_WAVE_MIN, (work_bound + per_simd - 1) / per_simd));
-    // whole waves per row: in a batch of equal lengths no wave then crosses from
+    const int64_t cap = one_per_simd && per_simd > 0 ? per_simd : resident;
+    const int64_t even = std::max<int64_t>(1, std::min((work_bound + per_wave - 1) / per_wave, cap));
+    if (!whole_rows) return {even, even};
+    // Whole waves per row: in a batch of equal lengths no wave then crosses from
     // one row into the next, which costs it a second start and both rows a
     // merge (32/8 heads, D 128, kernel us: 1 x 700 tokens 16.0 -> 12.3, 1 x 4000
-    // 32.0 -> 16.7, 8 x 1000 19.1 -> 13.8, 8 x 2500 30.1 -> 20.7; lengths spread
-    // over 1 : 32 within a few percent)
-    int64_t nw = whole_rows ? num_seqs * hkv * ((max_blocks + per_wave - 1) / per_wave)
-                            : (work_bound + per_wave - 1) / per_wave;
-    const int64_t cap = one_per_simd && per_simd > 0 ? per_simd : resident;
-    if (nw > cap) nw = cap;
-    return nw < 1 ? 1 : nw;
+    // 32.0 -> 16.7, 8 x 1000 19.1 -> 13.8, 8 x 2500 30.1 -> 20.7).  Not where the cap cuts
+    // them, nor where they alone would put a second wave on some SIMDs (FP8, 24 x
+    // 4000 tokens, 32/4 heads, 1000 -> 1056 waves: 52.8 -> 56.3 us, lengths within 1 : 2
+    // 36.1 -> 51.4); rows of one wave gain either way (FP8, 160 x 48 tokens, 32/16 heads,
+    // 23.4 -> 16.7).
+    // Mixed lengths put cuts inside rows whatever the count; up to 5 waves a row the
+    // more shares gain 1 to 20%, past that they lose as often (16/4 heads, 3 x 2000-4000
+    // tokens, 375 -> 384 waves 26.2 -> 34.3), or sit on a SIMD's second slot.
+    const int64_t per_row = (max_blocks + per_wave - 1) / per_wave;
+    const int64_t whole = std::max<int64_t>(1, std::min(rows * per_row, cap));
+    const bool fits = rows * per_row <= cap, crosses = even <= per_simd && whole > per_simd;
+    const int64_t waves = (fits && !crosses) || per_row == 1 ? whole : even;
+    const bool more = per_row <= 5 && !crosses && (fits || one_per_simd);
+    return {waves, waves == whole && more ? whole : even};
 }
 
 // Stream-mode workspace: arrival counters at offset 0, one per wave the device
@@ -1605,8 +1625,10 @@ int32_t decode_impl(void* out, const void* q, const void* kc, const void* vc, co
         if (max_waves < res) return (int32_t)hipErrorInvalidDevice;
         const bool fp8_kv = kv_dtype == KIND_FP8_E4M3 || kv_dtype == KIND_FP8_E5M2;
         auto waves = [&](bool whole_rows) {
-            plan.num_waves = static_cast<int32_t>(
-                stream_waves(num_seqs, hkv, maxb, res, 4 * int64_t(device_cus()), !fp8_kv, whole_rows));
+            const StreamWaves sw =
+                stream_waves(num_seqs, hkv, maxb, res, 4 * int64_t(device_cus()), !fp8_kv, whole_rows);
+            plan.num_waves = static_cast<int32_t>(sw.waves);
+            plan.mixed_waves = static_cast<int32_t>(sw.mixed);
             plan.max_waves = max_waves;
             plan.ws_bytes = plan.num_waves > 1 ? stream_ws_bytes(max_waves, plan.num_waves, G, d) : 0;
         };
@@ -1673,12 +1695,12 @@ int32_t decode_impl(void* out, const void* q, const void* kc, const void* vc, co
                 // capturing: scratch of a larger call may still hold equal shares
                 const bool fp8_kv = kv_dtype == KIND_FP8_E4M3 || kv_dtype == KIND_FP8_E5M2;
                 const int64_t nw = stream_waves(num_seqs, hkv, maxb, resident_waves(kern.stream, 1),
-                                                4 * int64_t(device_cus()), !fp8_kv, false);
+                                                4 * int64_t(device_cus()), !fp8_kv, false).waves;
                 const int64_t bytes = stream_ws_bytes(plan.max_waves, nw, G, d);
                 rc = g_workspaces.get(stream, role, bytes, true, &ws);
                 if (rc) return rc;
                 if (ws) {
-                    plan.num_waves = static_cast<int32_t>(nw);
+                    plan.num_waves = plan.mixed_waves = static_cast<int32_t>(nw);
                     plan.ws_bytes = bytes;
                 }
             }
@@ -1693,6 +1715,7 @@ int32_t decode_impl(void* out, const void* q, const void* kc, const void* vc, co
     a.part_chunks = plan.part_chunks;
     a.max_parts = plan.max_parts;
     a.num_waves = plan.num_waves;
+    a.mixed_waves = plan.mixed_waves;
     if (plan.ws_bytes > 0) {
         if (plan.mode == Mode::Stream) {
             a.arrivals = static_cast<uint32_t*>(ws);
@@ -1922,10 +1945,12 @@ int32_t mixed_impl(void* p_out, const void* p_q, const int32_t* p_bt, const int3
     const int64_t dpw = fp8 ? MIXED_DECODE_WAVES_FP8 : MIXED_DECODE_WAVES;
     const int max_waves = max_resident_waves();
     if (max_waves <= 0) return (int32_t)hipErrorInvalidDevice;
-    int64_t nw = 0, ws_bytes = 0;
+    int64_t nw = 0, mixed_nw = 0, ws_bytes = 0;
     auto plan_waves = [&](bool whole_rows) {
-        nw = std::min<int64_t>(
-            max_waves, stream_waves(d_num_seqs, hkv, d_maxb, dpw * free_cus, 4 * free_cus, dpw <= 4, whole_rows));
+        const StreamWaves sw =
+            stream_waves(d_num_seqs, hkv, d_maxb, dpw * free_cus, 4 * free_cus, dpw <= 4, whole_rows);
+        nw = std::min<int64_t>(max_waves, sw.waves);
+        mixed_nw = std::min<int64_t>(max_waves, sw.mixed);
         ws_bytes = nw > 1 ? stream_ws_bytes(max_waves, nw, G, d) : 0;
     };
     plan_waves(true);
@@ -1936,8 +1961,8 @@ int32_t mixed_impl(void* p_out, const void* p_q, const int32_t* p_bt, const int3
         if (rc) return rc;
         if (!ws) {
             // capturing: scratch of a larger step may still hold equal shares
-            // (whole rows of 24 sequences want more waves than those of 25: 960
-            // against 800 on 200 CUs, FP8, 128-block tables)
+            // (whole rows of 54 sequences want more waves than 55 of them take: 1728
+            // against 1375 on 216 CUs, FP8, 8 kv heads, 25-block tables)
             plan_waves(false);
             if (ws_bytes > 0) {
                 rc = g_workspaces.get(stream, WS_DECODE_STREAM, ws_bytes, true, &ws);
@@ -1960,6 +1985,7 @@ int32_t mixed_impl(void* p_out, const void* p_q, const int32_t* p_bt, const int3
     da.s_scale = scale * LOG2E * (fp8 ? k_scale : 1.0f);
     da.v_scale = fp8 ? v_scale : 1.0f;
     da.num_waves = static_cast<int32_t>(nw);
+    da.mixed_waves = static_cast<int32_t>(mixed_nw);
     if (ws_bytes > 0) {
         da.arrivals = static_cast<uint32_t*>(ws);
         da.part_out = reinterpret_cast<float*>(static_cast<char*>(ws) + stream_counter_bytes(max_waves));
@@ -2124,7 +2150,7 @@ int64_t rllm_paged_attention_decode_workspace_size(int64_t num_seqs, int64_t num
         if (res <= 0) return -1;
         // an upper bound over the cache dtypes (FP8 caches may take more waves)
         const int64_t nw =
-            stream_waves(num_seqs, num_kv_heads, max_num_blocks_per_seq, res, 4 * int64_t(device_cus()), false);
+            stream_waves(num_seqs, num_kv_heads, max_num_blocks_per_seq, res, 4 * int64_t(device_cus()), false).waves;
         return nw > 1 ? stream_ws_bytes(res, nw, num_q_heads / num_kv_heads, head_dim) : 0;
     }
     Plan plan;

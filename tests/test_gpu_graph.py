@@ -464,37 +464,37 @@ def _graph_nodes(g):
 
 
 def test_mixed_step_captured_after_a_larger_one_stays_one_launch(dev):
-    """Whole rows of 24 sequences want more stream waves, and scratch, than those of
-    25 (64/8 heads, FP8, 128-block tables, 56 prefill workgroups).  After an eager
-    step of 25 a captured step of 24 runs equal shares in the same one launch, not
-    the two groups in series."""
-    hq, hkv, d, maxb, T = 64, 8, 128, 128, 200
+    """Whole rows of 54 sequences want more stream waves, and scratch, than 55 take
+    (64/8 heads, FP8, 25-block tables, 40 prefill workgroups).  After an eager step
+    of 55 a captured step of 54 runs equal shares in the same one launch, not the
+    two groups in series."""
+    hq, hkv, d, maxb, T = 64, 8, 128, 25, 130
     gen = torch.Generator(device=dev)
     gen.manual_seed(11)
     rng = np.random.default_rng(11)
     kc, vc = (torch.randint(0, 96, (400, hkv, d, 16), generator=gen, device=dev, dtype=torch.uint8) for _ in range(2))
-    pq, dq = (torch.randn((n, hq, d), generator=gen, device=dev, dtype=torch.bfloat16) for n in (T, 25))
+    pq, dq = (torch.randn((n, hq, d), generator=gen, device=dev, dtype=torch.bfloat16) for n in (T, 55))
     pbt = ti(rng.permutation(400)[:40].reshape(1, 40).astype(np.int32), torch.int32, dev)
-    dbt = ti(rng.integers(0, 400, (25, maxb)).astype(np.int32), torch.int32, dev)
+    dbt = ti(rng.integers(0, 400, (55, maxb)).astype(np.int32), torch.int32, dev)
     psl, qsl = ti(np.array([600], np.int32), torch.int32, dev), ti(np.array([0, T], np.int32), torch.int32, dev)
-    dsl = ti(rng.integers(1, 16 * maxb, 25).astype(np.int32), torch.int32, dev)
+    dsl = ti(rng.integers(1, 16 * maxb, 55).astype(np.int32), torch.int32, dev)
     opt = dict(kv_dtype=rllm_amd.DTYPE_FP8_E4M3, k_scale=0.02, v_scale=0.02, validate=False)
 
     def call(n, outs):
         ops.paged_mixed(pq, pbt, psl, qsl, dq[:n], dbt[:n], dsl[:n], kc, vc, 0.1, prefill_out=outs[0],
                         decode_out=outs[1], **opt)
 
-    log_case("mixed step of 24 captured after 25")
-    eager, outs = ([torch.zeros_like(pq), torch.zeros_like(dq[:24])] for _ in range(2))
-    call(24, eager)
+    log_case("mixed step of 54 captured after 55")
+    eager, outs = ([torch.zeros_like(pq), torch.zeros_like(dq[:54])] for _ in range(2))
+    call(54, eager)
     torch.cuda.synchronize()
     with RawStream() as st:
         with torch.cuda.stream(st):
-            call(25, [torch.empty_like(pq), torch.empty_like(dq)])
+            call(55, [torch.empty_like(pq), torch.empty_like(dq)])
         torch.cuda.synchronize()
         g = torch.cuda.CUDAGraph(keep_graph=True)
         with torch.cuda.graph(g, stream=st):
-            call(24, outs)
+            call(54, outs)
         assert _graph_nodes(g) == 1
         g.instantiate()
         for r in range(3):
@@ -506,7 +506,7 @@ def test_mixed_step_captured_after_a_larger_one_stays_one_launch(dev):
             torch.cuda.synchronize()
             assert torch.equal(outs[0], eager[0]), f"replay {r}"
             assert_close(f32(outs[1]), f32(eager[1]), TOL_FP8, f"replay {r}")
-            call(24, [torch.empty_like(pq), torch.empty_like(dq[:24])])
+            call(54, [torch.empty_like(pq), torch.empty_like(dq[:54])])
 
 
 @pytest.mark.parametrize("B", [8, 40])
